@@ -37,44 +37,14 @@
 #include <type_traits>
 
 #include "df_common.hpp"
+#include "gemm_common.hpp"
 #include "gemm_sched.hpp"
 
 namespace dfk {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-
 constexpr int kBK = 128;              // bytes of K per step = one MFMA depth
 constexpr int kLdsStride = kBK + 16;  // padded LDS row (bytes)
 constexpr int kGroupM = 8;
-
-template <typename T> struct OutCvt;
-template <> struct OutCvt<float> {
-    static __device__ __forceinline__ float cvt(float v) { return v; }
-};
-template <> struct OutCvt<uint16_t> {  // bf16 bits
-    static __device__ __forceinline__ uint16_t cvt(float v) { return (uint16_t)f32_to_bf16_rne(v); }
-};
-template <> struct OutCvt<f16_t> {
-    static __device__ __forceinline__ f16_t cvt(float v) { return f16_t{(uint16_t)f32_to_f16_rne(v)}; }
-};
-__device__ __forceinline__ float bias_ld(const float* b, int i) { return b[i]; }
-__device__ __forceinline__ float bias_ld(const uint16_t* b, int i) { return bf16_to_f32(b[i]); }
-__device__ __forceinline__ float bias_ld(const f16_t* b, int i) { return f16_to_f32(b[i].bits); }
-
-// 4 consecutive outputs of one row: one 16-byte (fp32) or 8-byte (bf16) store
-__device__ __forceinline__ void store4(float* p, const float* v) {
-    *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
-}
-__device__ __forceinline__ void store4(uint16_t* p, const float* v) {
-    *reinterpret_cast<u32x2*>(p) = u32x2{f32_to_bf16_rne(v[0]) | (f32_to_bf16_rne(v[1]) << 16),
-                                        f32_to_bf16_rne(v[2]) | (f32_to_bf16_rne(v[3]) << 16)};
-}
-__device__ __forceinline__ void store4(f16_t* p, const float* v) {
-    *reinterpret_cast<u32x2*>(p) = u32x2{f32_to_f16_rne(v[0]) | (f32_to_f16_rne(v[1]) << 16),
-                                        f32_to_f16_rne(v[2]) | (f32_to_f16_rne(v[3]) << 16)};
-}
 
 __device__ __forceinline__ v8i lds_frag(const uint8_t* p) {
     const u32x4 lo = *reinterpret_cast<const u32x4*>(p);
@@ -1134,16 +1104,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     }
 }
 
-struct GemmArgs {
-    const uint8_t* A; int lda;
-    const uint8_t* B; int ldb;
-    int M, N, K;
-    const float* sa; const float* sb;
-    const void* bias; void* C; int ldc;
-    float* ws; size_t ws_bytes;
-    hipStream_t st;
-};
-
 // Launch plan: tile configuration and split-K factor from a rounds cost
 // model.  A 256x256 block (8 waves) occupies a CU alone: 256 tiles per
 // round.  128x128 blocks (4 waves) run two per CU: 512 per round, each
@@ -1318,11 +1278,13 @@ static void launch_persistent_narrow(const GemmArgs& g, int grid) {
 // faster there), while the GPT-2 XL shapes at 16384 tokens keep 256x256
 // tiles (narrow ones 13-40% slower).
 constexpr double kNarrowStep = 0.6, kNarrowOverhead = 2.0;
+constexpr double kReduceLaunch = 2.0;
 
 // The kernel one NT GEMM call runs (df_fp8_gemm_nt_plan reports it): the
 // persistent kernel when its offsets fit (split into K-slice units when the
 // output has fewer tiles than CUs and a workspace allows it; its 256x128
-// tiles when the rounds cost model puts them 3% below), otherwise the
+// tiles, or the small tiles of gemm_small.hip, when the rounds cost model
+// puts them 3% below), otherwise the
 // tiled kernels -- LDS-DMA when both operands fit a 32-bit buffer range,
 // register-staged beyond -- with 256x256 or 128x128 blocks and split-K from
 // plan_gemm.  Every launch below follows this plan.
@@ -1331,6 +1293,7 @@ struct NtPlan {
     int split;  // K slices (1 = unsplit)
     int L;      // persistent split: DMA steps per slice
     int grid;   // persistent: blocks
+    SmallPlan small{0, 0, 0, 0.0};  // waves > 0: gemm_small.hip's tiles (kind PERSISTENT_NARROW, split = waves)
 };
 
 static NtPlan nt_plan(const GemmArgs& g) {
@@ -1352,6 +1315,11 @@ static NtPlan nt_plan(const GemmArgs& g) {
             wcost = ps.cost;
         }
         const double ncost = (double)((tiles_nw + cus - 1) / cus) * (nk * kNarrowStep + kNarrowOverhead);
+        // a split plan's second launch (the slice reduce) costs kReduceLaunch
+        // steps that the choice between split and unsplit does not see
+        const SmallPlan sm = small_plan(g.M, g.N, g.K, cus);
+        if (sm.cost < std::min(ncost, wcost + (wide.split > 1 ? kReduceLaunch : 0.0)) * 0.97)
+            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, sm.waves, 0, 0, sm};
         if (ncost < wcost * 0.97)
             return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, 1, 0, (int)std::min<int64_t>(tiles_nw, cus)};
         return wide;
@@ -1370,8 +1338,12 @@ static NtPlan nt_plan(const GemmArgs& g) {
 }
 
 template <int FA, int FB, typename OutT, typename BiasT>
-static void launch_shape(const GemmArgs& g) {
+static void launch_shape(const GemmArgs& g, int bias_dtype, int c_dtype) {
     const NtPlan p = nt_plan(g);
+    if (p.small.waves) {
+        launch_small(p.small, FA, FB, bias_dtype, c_dtype, g);
+        return;
+    }
     if (p.kind == DF_GEMM_KERNEL_PERSISTENT_NARROW) {
         launch_persistent_narrow<FA, FB, OutT, BiasT>(g, p.grid);
         return;
@@ -1420,9 +1392,10 @@ static GroupPlan grouped_plan(const GemmArgs& dw, const GemmArgs& dx, size_t ws_
     const double red_steps_per_byte = 2.0 / 10e6;
     const int nk0 = (dw.K + kPKB - 1) / kPKB, nk1 = (dx.K + kPKB - 1) / kPKB;
     // Where df_fp8_gemm_bwd_dx, given this workspace, cuts dX's reduction into
-    // K slices (a small dX with a long reduction), dX is left to that call:
-    // the grouped launch never slices dX, and this keeps dX bit-identical
-    // between the two entry points.
+    // K slices (a small dX with a long reduction, or the small tiles, whose
+    // waves share the reduction), dX is left to that call: the grouped launch
+    // never slices dX, and this keeps dX bit-identical between the two entry
+    // points.
     GemmArgs dxs = dx;
     dxs.ws = ws_bytes ? reinterpret_cast<float*>(uintptr_t{16}) : nullptr;  // only its presence is read
     dxs.ws_bytes = ws_bytes;
@@ -1506,14 +1479,14 @@ static void dispatch_out(const GemmArgs& g, int bias_dtype, int c_dtype) {
     const bool bf16_bias = g.bias && bias_dtype == DF_DTYPE_BFLOAT16;
     const bool f16_bias = g.bias && bias_dtype == DF_DTYPE_HALF;
     if (c_dtype == DF_DTYPE_FLOAT32) {
-        if (bf16_bias) launch_shape<FA, FB, float, uint16_t>(g);
-        else launch_shape<FA, FB, float, float>(g);
+        if (bf16_bias) launch_shape<FA, FB, float, uint16_t>(g, bias_dtype, c_dtype);
+        else launch_shape<FA, FB, float, float>(g, bias_dtype, c_dtype);
     } else if (c_dtype == DF_DTYPE_HALF) {
-        if (f16_bias) launch_shape<FA, FB, f16_t, f16_t>(g);
-        else launch_shape<FA, FB, f16_t, float>(g);
+        if (f16_bias) launch_shape<FA, FB, f16_t, f16_t>(g, bias_dtype, c_dtype);
+        else launch_shape<FA, FB, f16_t, float>(g, bias_dtype, c_dtype);
     } else {
-        if (bf16_bias) launch_shape<FA, FB, uint16_t, uint16_t>(g);
-        else launch_shape<FA, FB, uint16_t, float>(g);
+        if (bf16_bias) launch_shape<FA, FB, uint16_t, uint16_t>(g, bias_dtype, c_dtype);
+        else launch_shape<FA, FB, uint16_t, float>(g, bias_dtype, c_dtype);
     }
 }
 

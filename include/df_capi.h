@@ -313,8 +313,9 @@ int df_fp8_gemm_nt(int fmt_a, const uint8_t* A, int lda,
  * kernel takes every call whose operands fit its 32-bit buffer offsets
  * (M*lda and N*ldb below 2^31, lda and ldb below 2^23) and whose bias is
  * 4-byte aligned, with 256x256 tiles or, where its rounds cost model
- * prefers them, 256x128 tiles (PERSISTENT_NARROW); the tiled kernels take
- * the rest, with LDS-DMA operand
+ * prefers them, narrower ones (PERSISTENT_NARROW: 256x128 with split 1, or
+ * 16x16 and 32x32 tiles whose `split` waves share the K steps and add up
+ * within the block); the tiled kernels take the rest, with LDS-DMA operand
  * loads while M*lda and N*ldb stay below 2^31 and register-staged loads
  * beyond.  Same plan as the reference-facing calls below; no reference
  * counterpart (the reference has one kernel per GEMM). */
