@@ -24,6 +24,29 @@ constexpr int kMaxReduceBlocks = 2048;  // partials in the absmax workspace
 // partials, so fewer than kMaxReduceBlocks (512: 2 KiB per tile block, and
 // still enough blocks for the absmax pass to stream at full rate)
 constexpr int kJitParts = 512;
+// df_quantize_2d_jit inputs of at most this many bytes run in one launch: each
+// tile block reads all of x for the absmax (one chunk of kU loads per thread)
+// instead of folding the partials of a pass before it.  8 x 1600 bf16 (25 KB):
+// 6.3 us against 8.4 with the separate pass; beyond one chunk the blocks' scans
+// cost what the launch saves (40 x 1000, 80 KB: 8.5 against 9.0; 8 x 6400,
+// 102 KB: 8.8 against 8.5; 64 x 1600, 205 KB: 11.3 against 8.5).
+constexpr int64_t kJitScanBytes = 32 << 10;
+
+// plain or non-temporal (NT) accesses.  The flat kernels store
+// non-temporal (NTS) when their output starts on a 128-byte boundary: every
+// wave store then covers whole cache lines.  A misaligned output takes plain
+// stores, so no line is assembled from several non-temporal partial writes
+// of neighbouring blocks.
+template <bool NT, typename T> __device__ __forceinline__ T ld_nt(const T* p) {
+    if (NT) return __builtin_nontemporal_load(p);
+    return *p;
+}
+template <bool NT, typename T> __device__ __forceinline__ void st_nt(T* p, const T v) {
+    if (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
 
 // ------------------------------------------------------------------ absmax --
 // (fold_f32 and fold_bf16x2, the binary32 and bf16-pair folds, are in df_common.hpp)
@@ -59,108 +82,70 @@ constexpr int64_t kChunkVec = (int64_t)kThreads * kU;
 // (at 2, 5.83-6.08).
 constexpr int kUQuantF32 = 2, kUQuantBf16 = 4, kUDeqF32 = 2, kUDeqBf16 = 1;
 
-// Stage 1 bodies: the block's maximum over its chunks (block bi of nb
-// blocks walking the chunks with a stride of nb).  |x| bit patterns, NaN
-// and infinities skipped (fold_*).
-__device__ __forceinline__ uint32_t absmax_f32_block(const float* __restrict__ x, int64_t n, int bi, int nb) {
-    uint32_t m = 0;
-    const int64_t nvec = n >> 2;
-    const u32x4* xv = reinterpret_cast<const u32x4*>(x);
-    for (int64_t base = (int64_t)bi * kChunkVec; base < nvec; base += (int64_t)nb * kChunkVec) {
-        if (base + kChunkVec <= nvec) {
-            u32x4 v[kU];
-#pragma unroll
-            for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load(xv + base + u * kThreads + threadIdx.x);
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                m = fold_f32(m, v[u].x); m = fold_f32(m, v[u].y); m = fold_f32(m, v[u].z); m = fold_f32(m, v[u].w);
-            }
-        } else {
-            for (int64_t i = base + threadIdx.x; i < nvec; i += kThreads) {
-                const u32x4 v = xv[i];
-                m = fold_f32(m, v.x); m = fold_f32(m, v.y); m = fold_f32(m, v.z); m = fold_f32(m, v.w);
-            }
-        }
-    }
-    if (bi == 0 && threadIdx.x < (n & 3))
-        m = fold_f32(m, __float_as_uint(x[(nvec << 2) + threadIdx.x]));
-    return block_max_u32(m);
-}
-
-// bf16: 16-byte loads hold 8 values.
-__device__ __forceinline__ uint32_t absmax_bf16_block(const uint16_t* __restrict__ x, int64_t n, int bi, int nb) {
-    uint32_t m = 0;
-    const int64_t nvec = n >> 3;
-    const u32x4* xv = reinterpret_cast<const u32x4*>(x);
-    for (int64_t base = (int64_t)bi * kChunkVec; base < nvec; base += (int64_t)nb * kChunkVec) {
-        if (base + kChunkVec <= nvec) {
-            u32x4 v[kU];
-#pragma unroll
-            for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load(xv + base + u * kThreads + threadIdx.x);
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                m = fold_bf16x2(m, v[u].x); m = fold_bf16x2(m, v[u].y);
-                m = fold_bf16x2(m, v[u].z); m = fold_bf16x2(m, v[u].w);
-            }
-        } else {
-            for (int64_t i = base + threadIdx.x; i < nvec; i += kThreads) {
-                const u32x4 v = xv[i];
-                m = fold_bf16x2(m, v.x); m = fold_bf16x2(m, v.y); m = fold_bf16x2(m, v.z); m = fold_bf16x2(m, v.w);
-            }
-        }
-    }
-    if (bi == 0 && threadIdx.x < (n & 7))
-        m = fold_f32(m, (uint32_t)x[(nvec << 3) + threadIdx.x] << 16);
-    return block_max_u32(m);
-}
-
-// binary16: 16-byte loads hold 8 values, each widened exactly.
+// Stage 1 body: the block's maximum over its chunks (block bi of nb blocks
+// walking the chunks with a stride of nb).  |x| bit patterns, NaN and
+// infinities skipped (fold_*).  InT: float, uint16_t (bf16) or f16_t.
 __device__ __forceinline__ uint32_t fold_f16x2(uint32_t m, uint32_t w) {
     m = fold_f32(m, __float_as_uint(f16_to_f32(w & 0xFFFFu)));
     return fold_f32(m, __float_as_uint(f16_to_f32(w >> 16)));
 }
-__device__ __forceinline__ uint32_t absmax_f16_block(const uint16_t* __restrict__ x, int64_t n, int bi, int nb) {
-    uint32_t m = 0;
-    const int64_t nvec = n >> 3;
-    const u32x4* xv = reinterpret_cast<const u32x4*>(x);
-    for (int64_t base = (int64_t)bi * kChunkVec; base < nvec; base += (int64_t)nb * kChunkVec) {
-        if (base + kChunkVec <= nvec) {
-            u32x4 v[kU];
-#pragma unroll
-            for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load(xv + base + u * kThreads + threadIdx.x);
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                m = fold_f16x2(m, v[u].x); m = fold_f16x2(m, v[u].y);
-                m = fold_f16x2(m, v[u].z); m = fold_f16x2(m, v[u].w);
-            }
-        } else {
-            for (int64_t i = base + threadIdx.x; i < nvec; i += kThreads) {
-                const u32x4 v = xv[i];
-                m = fold_f16x2(m, v.x); m = fold_f16x2(m, v.y); m = fold_f16x2(m, v.z); m = fold_f16x2(m, v.w);
-            }
-        }
+template <typename InT> __device__ __forceinline__ uint32_t fold_vec(uint32_t m, const u32x4 v) {
+    if constexpr (std::is_same<InT, float>::value) {
+        m = fold_f32(m, v.x); m = fold_f32(m, v.y); m = fold_f32(m, v.z); return fold_f32(m, v.w);
+    } else if constexpr (std::is_same<InT, f16_t>::value) {
+        m = fold_f16x2(m, v.x); m = fold_f16x2(m, v.y); m = fold_f16x2(m, v.z); return fold_f16x2(m, v.w);
+    } else {
+        m = fold_bf16x2(m, v.x); m = fold_bf16x2(m, v.y); m = fold_bf16x2(m, v.z); return fold_bf16x2(m, v.w);
     }
-    if (bi == 0 && threadIdx.x < (n & 7))
-        m = fold_f32(m, __float_as_uint(f16_to_f32(x[(nvec << 3) + threadIdx.x])));
+}
+template <typename InT> __device__ __forceinline__ uint32_t fold_one(uint32_t m, const InT* p) {
+    if constexpr (std::is_same<InT, float>::value) return fold_f32(m, __float_as_uint(*p));
+    else if constexpr (std::is_same<InT, f16_t>::value) return fold_f32(m, __float_as_uint(f16_to_f32(p->bits)));
+    else return fold_f32(m, (uint32_t)*p << 16);
+}
+
+template <typename InT, bool NT = true>
+__device__ __forceinline__ uint32_t absmax_block(const InT* __restrict__ x, int64_t n, int bi, int nb) {
+    constexpr int E = 16 / (int)sizeof(InT);
+    uint32_t m = 0;
+    const int64_t nvec = n / E;
+    const u32x4* xv = reinterpret_cast<const u32x4*>(x);
+    int64_t base = (int64_t)bi * kChunkVec;
+    for (; base + kChunkVec <= nvec; base += (int64_t)nb * kChunkVec) {
+        u32x4 v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) v[u] = ld_nt<NT>(xv + base + u * kThreads + threadIdx.x);
+        __builtin_amdgcn_sched_barrier(0);  // no fold before the last load has left
+#pragma unroll
+        for (int u = 0; u < kU; ++u) m = fold_vec<InT>(m, v[u]);
+    }
+    if (base < nvec) {
+        // the last, partial chunk: loads past it take the last vector again
+        // (a maximum does not mind), so all are in flight together
+        u32x4 v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) v[u] = xv[min(base + u * kThreads + (int64_t)threadIdx.x, nvec - 1)];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) m = fold_vec<InT>(m, v[u]);
+    }
+    if (bi == 0 && threadIdx.x < n - nvec * E) m = fold_one<InT>(m, x + nvec * E + threadIdx.x);
     return block_max_u32(m);
 }
 
 // Stage 1: one partial maximum per block.
 __global__ __launch_bounds__(kThreads) void absmax_f32_stage1(const float* __restrict__ x, int64_t n,
                                                                uint32_t* __restrict__ partial) {
-    const uint32_t m = absmax_f32_block(x, n, blockIdx.x, gridDim.x);
+    const uint32_t m = absmax_block<float>(x, n, blockIdx.x, gridDim.x);
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
-
 __global__ __launch_bounds__(kThreads) void absmax_bf16_stage1(const uint16_t* __restrict__ x, int64_t n,
-                                                                uint32_t* __restrict__ partial) {
-    const uint32_t m = absmax_bf16_block(x, n, blockIdx.x, gridDim.x);
+                                                               uint32_t* __restrict__ partial) {
+    const uint32_t m = absmax_block<uint16_t>(x, n, blockIdx.x, gridDim.x);
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
-
-__global__ __launch_bounds__(kThreads) void absmax_f16_stage1(const uint16_t* __restrict__ x, int64_t n,
+__global__ __launch_bounds__(kThreads) void absmax_f16_stage1(const f16_t* __restrict__ x, int64_t n,
                                                                uint32_t* __restrict__ partial) {
-    const uint32_t m = absmax_f16_block(x, n, blockIdx.x, gridDim.x);
+    const uint32_t m = absmax_block<f16_t>(x, n, blockIdx.x, gridDim.x);
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
@@ -217,12 +202,10 @@ struct JitScale {
     float* scale_out = nullptr;
 };
 
-__device__ __forceinline__ float jit_block_scale(const uint32_t* __restrict__ parts, int nparts, int fmt,
-                                                 float* __restrict__ absmax_out, float* __restrict__ scale_out,
-                                                 bool writer) {
+__device__ __forceinline__ float block_scale(uint32_t m, int fmt, float* __restrict__ absmax_out,
+                                             float* __restrict__ scale_out, bool writer) {
     __shared__ float s_scale;
-    const uint32_t m = block_max_u32(fold_parts(parts, nparts));
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0) {  // m: the block's maximum, valid in thread 0
         const float am = __uint_as_float(m), sc = scale_from_absmax(am, fmt);
         s_scale = sc;
         if (writer) {
@@ -234,6 +217,12 @@ __device__ __forceinline__ float jit_block_scale(const uint32_t* __restrict__ pa
     return s_scale;
 }
 
+__device__ __forceinline__ float jit_block_scale(const uint32_t* __restrict__ parts, int nparts, int fmt,
+                                                 float* __restrict__ absmax_out, float* __restrict__ scale_out,
+                                                 bool writer) {
+    return block_scale(block_max_u32(fold_parts(parts, nparts)), fmt, absmax_out, scale_out, writer);
+}
+
 __global__ void scale_kernel(const float* __restrict__ absmax, int fmt, float* __restrict__ scale) {
     if (threadIdx.x == 0) scale[0] = scale_from_absmax(absmax[0], fmt);
 }
@@ -241,22 +230,6 @@ __global__ void scale_kernel(const float* __restrict__ absmax, int fmt, float* _
 // ---------------------------------------------------------------- quantize --
 // x / s (correctly rounded: qdiv, contract D1), then the fp8 encoder
 // (encode2_hw: hardware round-to-nearest-even after saturation, NaN kept).
-
-// plain or non-temporal (NT) accesses.  The flat kernels store
-// non-temporal (NTS) when their output starts on a 128-byte boundary: every
-// wave store then covers whole cache lines.  A misaligned output takes plain
-// stores, so no line is assembled from several non-temporal partial writes
-// of neighbouring blocks.
-template <bool NT, typename T> __device__ __forceinline__ T ld_nt(const T* p) {
-    if (NT) return __builtin_nontemporal_load(p);
-    return *p;
-}
-template <bool NT, typename T> __device__ __forceinline__ void st_nt(T* p, const T v) {
-    if (NT)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
-}
 
 // fp32 -> fp8: a 16-byte load of 4 values -> a 4-byte store of 4 codes.
 template <int FMT, bool FAST, bool NTS>
@@ -570,6 +543,33 @@ template <> struct Ld<f16_t> {
     static __device__ __forceinline__ float one(const f16_t* p) { return f16_to_f32(p->bits); }
 };
 
+// 16 bytes from an address aligned to the element only (gfx950 reads global
+// memory at any alignment; the compiler emits the same 16-byte load)
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 ld16_any(const void* p) { return *static_cast<const u32x4_any*>(p); }
+
+// x[c .. c+E) of a row shorter than one chunk (cols < E), zeros past its end
+template <typename InT> __device__ __forceinline__ u32x4 ld_short(const InT* __restrict__ row, int c, int cols) {
+    constexpr int E = Ld<InT>::E;
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        if (c + e < cols) {
+            if constexpr (sizeof(InT) == 4) w[e & 3] = __builtin_bit_cast(uint32_t, row[c + e]);
+            else w[e >> 1] |= (uint32_t)__builtin_bit_cast(uint16_t, row[c + e]) << (16 * (e & 1));
+        }
+    }
+    return u32x4{w[0], w[1], w[2], w[3]};
+}
+
+// Drops the first by % 16 bytes (even) of a 16-byte chunk; zeros follow.
+__device__ __forceinline__ u32x4 drop_bytes(u32x4 w, int by) {
+    if (by & 8) w = u32x4{w.z, w.w, 0, 0};
+    if (by & 4) w = u32x4{w.y, w.z, w.w, 0};
+    if (by & 2) w = u32x4{(w.x >> 16) | (w.y << 16), (w.y >> 16) | (w.z << 16), (w.z >> 16) | (w.w << 16), w.w >> 16};
+    return w;
+}
+
 // ---------------------------------------------------------------- LayerNorm --
 // Row statistics and the per-element map of the reference's
 // layer_norm_forward_kernel (dnn/layers/layer_norm_layer.cu:26-63):
@@ -650,6 +650,7 @@ __device__ __forceinline__ void q2d_tile(const InT* __restrict__ x, int rows, in
     constexpr int TPR = kT2 / E;       // threads per tile row
     constexpr int RG = kThreads / TPR; // row groups
     constexpr int RPT = TR / RG;       // rows per thread (8 for bf16, 16 for fp32 at TR = 128)
+    constexpr int EB = 8;              // rows in flight on an edge
     static_assert(RPT % 4 == 0 && RPT <= 32, "4x4 byte transposes");
     static_assert(TR == 128 && (RPT == 8 || RPT == 16), "the tslot layout holds 128-row tiles, 8 or 16 rows a thread");
     const int r0 = by * TR, c0 = bx * kT2;  // tile (bx, by) of a grid nbx tiles wide
@@ -742,19 +743,41 @@ __device__ __forceinline__ void q2d_tile(const InT* __restrict__ x, int rows, in
             Ld<InT>::widen(raw[rr], v);
             row(rr, v);
         }
-    } else {
+    } else if (c >= cols) {  // a column group of padding: code 0
 #pragma unroll
         for (int rr = 0; rr < RPT; ++rr) {
             const int r = r0 + rg * RPT + rr;
-            float v[E];
-            if (r < rows && full) {
-                Ld<InT>::vec(x + (int64_t)r * ldx + c, v);
-            } else {
 #pragma unroll
-                for (int e = 0; e < E; ++e)
-                    v[e] = (r < rows && c + e < cols) ? Ld<InT>::one(x + (int64_t)r * ldx + c + e) : 0.0f;
+            for (int g = 0; g < E / 4; ++g) codes[rr][g] = 0;
+            if (CODES && q && r < rows && c < ldq) {
+                if (E == 8) *reinterpret_cast<u32x2*>(q + (int64_t)r * ldq + c) = u32x2{0, 0};
+                else *reinterpret_cast<uint32_t*>(q + (int64_t)r * ldq + c) = 0;
             }
-            row(rr, v);
+        }
+    } else {
+        // edge tiles, and rows that are not 16-byte aligned: EB rows in flight
+        // at a time (all RPT at once cost the main path its occupancy).  A
+        // chunk that runs past the row's end is read as the row's last E
+        // values, and those before column c are dropped.
+        const int over = c + E - cols, cl = over > 0 ? cols - E : c;
+        const int by = over > 0 && cols >= E ? over * (int)sizeof(InT) : 0;
+#pragma unroll
+        for (int r1 = 0; r1 < RPT; r1 += EB) {
+            u32x4 raw[EB];
+#pragma unroll
+            for (int rr = 0; rr < EB; ++rr) {
+                const int r = r0 + rg * RPT + r1 + rr;
+                raw[rr] = u32x4{0, 0, 0, 0};
+                if (r < rows)
+                    raw[rr] = cols >= E ? ld16_any(x + (int64_t)r * ldx + cl)
+                                        : ld_short<InT>(x + (int64_t)r * ldx, c, cols);
+            }
+#pragma unroll
+            for (int rr = 0; rr < EB; ++rr) {
+                float v[E];
+                Ld<InT>::widen(drop_bytes(raw[rr], by), v);
+                row(r1 + rr, v);
+            }
         }
     }
     if (CODES && qt) {
@@ -973,7 +996,8 @@ __global__ __launch_bounds__(kThreads) void amax_history_init_kernel(const float
 
 // JIT: the scale comes from the absmax partials in jit (jit_block_scale;
 // block (0, 0) writes absmax and scale), not from scale[0].
-template <typename InT, int FMT, bool COLSUM, bool CODES, bool AMAX, bool LN, bool JIT>
+// SCAN: a small x, whose absmax every block takes itself (kJitScanBytes).
+template <typename InT, int FMT, bool COLSUM, bool CODES, bool AMAX, bool LN, bool JIT, bool SCAN = false>
 __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int rows, int cols, int ldx, bool vec_ok,
                                                 const float* __restrict__ scale, uint8_t* __restrict__ q, int ldq,
                                                 uint8_t* __restrict__ qt, int ldqt, float* __restrict__ colpart,
@@ -984,11 +1008,15 @@ __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int r
     __shared__ __attribute__((aligned(16))) uint8_t tile[kT2 * kT2R];
     __shared__ float csum[COLSUM ? RG : 1][kT2];
     float sc = 1.0f;
-    if constexpr (JIT)
-        sc = jit_block_scale(jit.parts, jit.nparts, FMT, jit.absmax_out, jit.scale_out,
-                             blockIdx.x == 0 && blockIdx.y == 0);
-    else if constexpr (CODES)
-        sc = scale[0];
+    if constexpr (JIT) {
+        const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
+        if constexpr (SCAN)
+            sc = block_scale(absmax_block<InT, false>(x, (int64_t)rows * cols, 0, 1), FMT, jit.absmax_out,
+                             jit.scale_out, writer);
+        else
+            sc = jit_block_scale(jit.parts, jit.nparts, FMT, jit.absmax_out, jit.scale_out, writer);
+    }
+    if constexpr (CODES && !JIT) sc = scale[0];
     const QDiv d = make_qdiv(sc);
     if (!CODES || d.fast)
         q2d_tile<InT, FMT, COLSUM, CODES, AMAX, LN, true, AMAX && !LN, kT2R>(
@@ -1000,8 +1028,14 @@ __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int r
             blockIdx.y, gridDim.x);
 }
 
+// fp32 codes (column sums) alone: held to the five (six) waves per SIMD that
+// the registers allow (the compiler takes 102 and 87 where 82 and 80 do).
+constexpr int q2d_waves(bool f32, bool colsum, bool codes, bool amax, bool ln) {
+    return !f32 || amax || ln ? 1 : !codes ? 6 : colsum ? 1 : 5;
+}
 template <typename InT, int FMT, bool COLSUM, bool CODES, bool AMAX = false, bool LN = false>
-__global__ __launch_bounds__(kThreads) void quantize_2d_kernel(const InT* __restrict__ x, int rows,
+__global__ __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(q2d_waves(sizeof(InT) == 4, COLSUM, CODES, AMAX, LN)))) void quantize_2d_kernel(const InT* __restrict__ x, int rows,
                                                                 int cols, int ldx, bool vec_ok,
                                                                 const float* __restrict__ scale,
                                                                 uint8_t* __restrict__ q, int ldq,
@@ -1035,9 +1069,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
 }
 
 template <typename InT, int FMT, bool COLSUM>
+__global__ __launch_bounds__(kThreads) void quantize_2d_jit_scan_kernel(const InT* __restrict__ x, int rows, int cols,
+                                                                         bool vec_ok, uint8_t* __restrict__ q, int ldq,
+                                                                         uint8_t* __restrict__ qt, int ldqt,
+                                                                         float* __restrict__ colpart, JitScale jit) {
+    q2d_kernel_body<InT, FMT, COLSUM, true, false, false, true, true>(x, rows, cols, cols, vec_ok, nullptr, q, ldq, qt,
+                                                                      ldqt, colpart, nullptr, LnArgs(), jit);
+}
+
+template <typename InT, int FMT, bool COLSUM>
 static void launch_q2d_jit(dim3 grid, hipStream_t st, const InT* x, int rows, int cols, bool vec_ok, uint8_t* q,
                            int ldq, uint8_t* qt, int ldqt, float* colpart, const JitScale& jit) {
-    if constexpr (sizeof(InT) == 2 || !COLSUM)
+    if (!jit.nparts)
+        quantize_2d_jit_scan_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
+                                                                                  ldqt, colpart, jit);
+    else if constexpr (sizeof(InT) == 2 || !COLSUM)
         quantize_2d_jit_w5_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
                                                                                 ldqt, colpart, jit);
     else
@@ -1086,11 +1132,7 @@ __global__ __launch_bounds__(kThreads) void absmax_batch_stage1(const BatchArgs 
     const int t = batch_owner(B.blk_first, B.count, blockIdx.x);
     const int bi = blockIdx.x - B.blk_first[t], nb = B.blk_first[t + 1] - B.blk_first[t];
     const int64_t n = (int64_t)B.rows[t] * B.cols[t];
-    uint32_t m;
-    if constexpr (std::is_same<InT, float>::value)
-        m = absmax_f32_block(static_cast<const float*>(B.x[t]), n, bi, nb);
-    else
-        m = absmax_bf16_block(static_cast<const uint16_t*>(B.x[t]), n, bi, nb);
+    const uint32_t m = absmax_block<InT>(static_cast<const InT*>(B.x[t]), n, bi, nb);
     if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
@@ -1316,7 +1358,7 @@ static int launch_absmax_stage1(int in_dtype, const void* x, int64_t n, uint32_t
     else if (in_dtype == DF_DTYPE_BFLOAT16)
         absmax_bf16_stage1<<<blocks, kThreads, 0, st>>>(static_cast<const uint16_t*>(x), n, part);
     else
-        absmax_f16_stage1<<<blocks, kThreads, 0, st>>>(static_cast<const uint16_t*>(x), n, part);
+        absmax_f16_stage1<<<blocks, kThreads, 0, st>>>(static_cast<const f16_t*>(x), n, part);
     return blocks;
 }
 
@@ -1575,7 +1617,8 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
     JitScale J;
     if (jit) {
         uint32_t* jparts = reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + jit_off);
-        J.nparts = launch_absmax_stage1(in_dtype, x, (int64_t)rows * cols, jparts, st, kJitParts);
+        if ((int64_t)rows * cols * esz > kJitScanBytes)
+            J.nparts = launch_absmax_stage1(in_dtype, x, (int64_t)rows * cols, jparts, st, kJitParts);
         J.parts = jparts;
         J.absmax_out = jit_absmax;
         J.scale_out = const_cast<float*>(scale_dev);

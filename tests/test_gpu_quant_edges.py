@@ -1,0 +1,68 @@
+"""The 2-D quantize's edge loads (rows that are not 16-byte aligned, chunks
+that run past a row's end, rows shorter than a chunk, tiles partly or wholly
+of padding) and the one-launch form of the just-in-time quantize for small
+inputs, against the oracle: codes, transposed codes, their zero padding,
+absmax and scale bit for bit, column sums within binary32 summation error."""
+import numpy as np
+import pytest
+import torch
+
+import deepfuse_amd as df
+from deepfuse_amd import Fmt
+from oracle import pyoracle as orc
+
+pytestmark = pytest.mark.gpu
+
+F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+# one value, rows shorter than a 16-byte chunk, one value past / short of a
+# chunk and of a tile, 32 KB of input on, below and above (the one-launch form's limit)
+SHAPES = [(1, 1), (3, 3), (5, 7), (129, 5), (2, 9), (127, 129), (128, 127), (130, 136), (257, 131), (8, 1600),
+          (16, 1024), (16, 1025), (31, 264), (64, 128), (8, 1023), (300, 77)]
+
+
+def tensor(rows, cols, dt, dev, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, cols, generator=g) * 3
+    if rows * cols > 16:  # specials, one in the last row and column
+        flat = x.view(-1)
+        at = torch.randperm(rows * cols - 1, generator=g)[:5]
+        flat[at] = torch.tensor([float("nan"), float("inf"), float("-inf"), 0.0, -0.0])
+        flat[-1] = 11.5  # the absmax, in the last chunk
+    return x.to(dt).to(dev)
+
+
+def host(x):
+    return x.float().cpu().numpy()  # exact for the 2-byte types
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+@pytest.mark.parametrize("dt", [F32, BF16, F16])
+@pytest.mark.parametrize("fmt", [Fmt.E4M3, Fmt.E5M2])
+def test_edges(dev, rows, cols, dt, fmt):
+    x = tensor(rows, cols, dt, dev, rows * 1009 + cols)
+    h = host(x)
+    am, sc, q, qt, cs = df.quantize_2d_jit(x, fmt, want_qt=True, colsum=True)
+    s = orc.scale(orc.absmax(h), int(fmt))
+    assert am.item() == orc.absmax(h) and sc.item() == np.float32(s)
+    codes = orc.quantize(h, s, int(fmt))
+
+    def check(q, qt):
+        qh, th = q.cpu().numpy(), qt.cpu().numpy()
+        assert np.array_equal(qh[:, :cols], codes) and not qh[:, cols:].any()
+        assert np.array_equal(th[:, :rows], codes.T) and not th[:, rows:].any()
+
+    check(q, qt)
+    finite = np.isfinite(h).all(axis=0)
+    ref = h.astype(np.float64).sum(axis=0)
+    # binary32 sums of `rows` values: at most rows * 2^-24 of the sum of magnitudes
+    bound = rows * 2.0 ** -24 * np.abs(h.astype(np.float64)).sum(axis=0) + 1e-30
+    assert (np.abs(cs.cpu().numpy()[finite] - ref[finite]) <= bound[finite]).all()
+    # the same without column sums, the plain pass at that scale, and the
+    # rows of a wider matrix (a stride that is not a multiple of 16 bytes)
+    _, sc2, q2, qt2 = df.quantize_2d_jit(x, fmt, want_qt=True)
+    assert sc2.item() == sc.item()
+    check(q2, qt2)
+    check(*df.quantize_2d(x, sc, fmt, want_qt=True))
+    wide = torch.full((rows, cols + 3), float("nan"), dtype=dt, device=dev)
+    wide[:, :cols].copy_(x)
+    check(*df.quantize_2d(wide[:, :cols], sc, fmt, want_qt=True))
