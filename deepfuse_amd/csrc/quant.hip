@@ -98,6 +98,21 @@ template <typename InT> __device__ __forceinline__ uint32_t fold_vec(uint32_t m,
         m = fold_bf16x2(m, v.x); m = fold_bf16x2(m, v.y); m = fold_bf16x2(m, v.z); return fold_bf16x2(m, v.w);
     }
 }
+// the compare-free forms (df_common.hpp): three operations per dword
+template <typename InT> __device__ __forceinline__ uint32_t fold_vec_biased(uint32_t m, const u32x4 v) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (std::is_same<InT, float>::value) m = fold_f32_biased(m, v[i]);
+        else if constexpr (std::is_same<InT, f16_t>::value) m = fold_f16x2_biased(m, v[i]);
+        else m = fold_bf16x2_biased(m, v[i]);
+    }
+    return m;
+}
+template <typename InT> __device__ __forceinline__ uint32_t unbias(uint32_t m) {
+    if constexpr (std::is_same<InT, float>::value) return unbias_f32(m);
+    else if constexpr (std::is_same<InT, f16_t>::value) return unbias_f16x2(m);
+    else return unbias_bf16x2(m);
+}
 template <typename InT> __device__ __forceinline__ uint32_t fold_one(uint32_t m, const InT* p) {
     if constexpr (std::is_same<InT, float>::value) return fold_f32(m, __float_as_uint(*p));
     else if constexpr (std::is_same<InT, f16_t>::value) return fold_f32(m, __float_as_uint(f16_to_f32(p->bits)));
@@ -200,6 +215,11 @@ struct JitScale {
     int nparts = 0;
     float* absmax_out = nullptr;
     float* scale_out = nullptr;
+    // column sums: the partials of the absmax pass ([tile_rows][cols]) are
+    // added up into colsum by the first row of tile blocks (NULL: none)
+    const float* colpart = nullptr;
+    float* colsum = nullptr;
+    int tile_rows = 0;
 };
 
 __device__ __forceinline__ float block_scale(uint32_t m, int fmt, float* __restrict__ absmax_out,
@@ -994,6 +1014,116 @@ __global__ __launch_bounds__(kThreads) void amax_history_init_kernel(const float
 }
 
 
+// The absmax pass of a just-in-time quantize with column sums: the same
+// partial maxima as absmax_block, and on the way the fp32 column sums of every
+// 128-row tile, in the tile pass's order (a thread's rows in order, then the
+// row groups in order), so that the tile pass carries no sums: they cost it 37
+// registers, and it ran at five waves per SIMD instead of eight.  A block walks
+// tiles; the next tile's loads are on their way while it adds up this one.
+// With the sums left to this pass and their reduction to the first tile blocks
+// a call takes 33.8 us at 16384 x 1600 bf16 and 82.9 at 16384 x 4800, against
+// 39.4 and 90.0 with the sums in the tile pass and a reduce launch; 512 x 768
+// 10.0 against 10.7; 16384 x 6400 the same 121.
+template <typename InT>
+__global__ __launch_bounds__(kThreads) void absmax_colsum_stage1(const InT* __restrict__ x, int rows, int cols,
+                                                                  bool vec_ok, uint32_t* __restrict__ partial,
+                                                                  float* __restrict__ colpart) {
+    constexpr int E = Ld<InT>::E, TPR = kT2 / E, RG = kThreads / TPR, RPT = kT2R / RG;
+    __shared__ float csum[2][RG][kT2];
+    const int nbx = (cols + kT2 - 1) / kT2, nt = nbx * ((rows + kT2R - 1) / kT2R);
+    const int tc = (threadIdx.x % TPR) * E, rg = threadIdx.x / TPR;
+    auto load = [&](int t, u32x4* raw) __attribute__((always_inline)) {
+        const int by = t / nbx, c = (t - by * nbx) * kT2 + tc, r0 = by * kT2R + rg * RPT;
+        if (vec_ok && c + E <= cols && by * kT2R + kT2R <= rows) {
+#pragma unroll
+            for (int rr = 0; rr < RPT; ++rr)
+                raw[rr] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + (int64_t)(r0 + rr) * cols + c));
+        } else {
+            const int over = c + E - cols, cl = over > 0 ? cols - E : c;
+#pragma unroll
+            for (int rr = 0; rr < RPT; ++rr) {
+                raw[rr] = u32x4{0, 0, 0, 0};
+                if (r0 + rr < rows && c < cols)
+                    raw[rr] = cols >= E ? ld16_any(x + (int64_t)(r0 + rr) * cols + cl)
+                                        : ld_short<InT>(x + (int64_t)(r0 + rr) * cols, c, cols);
+            }
+            if (over > 0 && cols >= E) {
+#pragma unroll
+                for (int rr = 0; rr < RPT; ++rr) raw[rr] = drop_bytes(raw[rr], over * (int)sizeof(InT));
+            }
+        }
+    };
+    u32x4 cur[RPT], nxt[RPT];
+    uint32_t m = 0;
+    int t = blockIdx.x, b = 0;
+    if (t < nt) load(t, cur);
+    for (; t < nt; t += gridDim.x, b ^= 1) {
+        if (t + (int)gridDim.x < nt) load(t + gridDim.x, nxt);
+        __builtin_amdgcn_sched_barrier(0);  // the next tile's loads leave first
+        float cs[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) cs[e] = 0.0f;
+#pragma unroll
+        for (int rr = 0; rr < RPT; ++rr) {
+            float v[E];
+            Ld<InT>::widen(cur[rr], v);
+#pragma unroll
+            for (int e = 0; e < E; ++e) cs[e] += v[e];
+            m = fold_vec_biased<InT>(m, cur[rr]);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) csum[b][rg][tc + e] = cs[e];
+        __syncthreads();  // two buffers: the next tile's sums go into the other one
+        const int by = t / nbx, c0 = (t - by * nbx) * kT2;
+        if (threadIdx.x < kT2 && c0 + (int)threadIdx.x < cols) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int g = 0; g < RG; ++g) sum += csum[b][g][threadIdx.x];
+            colpart[(int64_t)by * cols + c0 + threadIdx.x] = sum;
+        }
+#pragma unroll
+        for (int rr = 0; rr < RPT; ++rr) cur[rr] = nxt[rr];
+    }
+    m = block_max_u32(unbias<InT>(m));
+    if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+// colsum_reduce_kernel's sums, in its order, of columns [c0, c0 + kT2) by one
+// block: four interleaved sums of tile rows, then those four in order.
+__device__ __forceinline__ void finish_colsum(const float* __restrict__ colpart, int tiles, int cols, int c0,
+                                              float* __restrict__ out) {
+    static_assert(kThreads == 2 * kT2, "two of the four sums per thread");
+    __shared__ float part[4][kT2];
+    const int k = threadIdx.x % kT2, c = c0 + k, w = threadIdx.x / kT2;
+    const float* p = colpart + (c < cols ? c : cols - 1);
+    float s[2] = {0.0f, 0.0f};
+    // sums w and w + 2, eight tile rows of each in flight (more would cost the
+    // tile pass its occupancy); a tile row past the last adds +0, which
+    // changes no sum (none is -0)
+#pragma unroll 1
+    for (int t0 = w; t0 < tiles; t0 += 32) {
+        float v[2][8];
+        const float* pt = p + (int64_t)t0 * cols;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                v[h][u] = t0 + 2 * h + 4 * u < tiles ? *pt : 0.0f;
+                pt += 2 * (int64_t)cols;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            s[0] += v[0][u];
+            s[1] += v[1][u];
+        }
+    }
+    part[w][k] = s[0];
+    part[w + 2][k] = s[1];
+    __syncthreads();
+    if (threadIdx.x < kT2 && c < cols) out[c] = ((part[0][k] + part[1][k]) + part[2][k]) + part[3][k];
+}
+
 // JIT: the scale comes from the absmax partials in jit (jit_block_scale;
 // block (0, 0) writes absmax and scale), not from scale[0].
 // SCAN: a small x, whose absmax every block takes itself (kJitScanBytes).
@@ -1006,7 +1136,9 @@ __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int r
     static_assert(!JIT || (CODES && !AMAX && !LN), "just-in-time scale: the plain code pass");
     constexpr int RG = kThreads / (kT2 / Ld<InT>::E);
     __shared__ __attribute__((aligned(16))) uint8_t tile[kT2 * kT2R];
-    __shared__ float csum[COLSUM ? RG : 1][kT2];
+    // a two-pass just-in-time call has its sums from the absmax pass
+    constexpr bool TILE_SUMS = COLSUM && !(JIT && !SCAN);
+    __shared__ float csum[TILE_SUMS ? RG : 1][kT2];
     float sc = 1.0f;
     if constexpr (JIT) {
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
@@ -1019,13 +1151,17 @@ __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int r
     if constexpr (CODES && !JIT) sc = scale[0];
     const QDiv d = make_qdiv(sc);
     if (!CODES || d.fast)
-        q2d_tile<InT, FMT, COLSUM, CODES, AMAX, LN, true, AMAX && !LN, kT2R>(
+        q2d_tile<InT, FMT, TILE_SUMS, CODES, AMAX, LN, true, AMAX && !LN, kT2R>(
             x, rows, cols, ldx, vec_ok, d, q, ldq, qt, ldqt, colpart, amaxpart, ln, tile, csum, blockIdx.x,
             blockIdx.y, gridDim.x);
     else
-        q2d_tile<InT, FMT, COLSUM, CODES, AMAX, LN, false, AMAX && !LN, kT2R>(
+        q2d_tile<InT, FMT, TILE_SUMS, CODES, AMAX, LN, false, AMAX && !LN, kT2R>(
             x, rows, cols, ldx, vec_ok, d, q, ldq, qt, ldqt, colpart, amaxpart, ln, tile, csum, blockIdx.x,
             blockIdx.y, gridDim.x);
+    if constexpr (COLSUM && !TILE_SUMS) {
+        if (blockIdx.y == 0 && jit.colsum)
+            finish_colsum(jit.colpart, jit.tile_rows, cols, blockIdx.x * kT2, jit.colsum);
+    }
 }
 
 // fp32 codes (column sums) alone: held to the five (six) waves per SIMD that
@@ -1047,27 +1183,18 @@ __global__ __launch_bounds__(kThreads)
                                                               colpart, amaxpart, ln, JitScale());
 }
 
-// The just-in-time pass (df_quantize_2d_jit), x contiguous.  The _w5 form
-// holds it to five waves per SIMD, the occupancy of the same pass without the
-// fold (the fold's registers are dead before the tile pass); fp32 with column
-// sums has four either way and takes the plain form.
-template <typename InT, int FMT, bool COLSUM>
-__global__ __launch_bounds__(kThreads) void quantize_2d_jit_kernel(const InT* __restrict__ x, int rows, int cols,
-                                                                    bool vec_ok, uint8_t* __restrict__ q, int ldq,
-                                                                    uint8_t* __restrict__ qt, int ldqt,
-                                                                    float* __restrict__ colpart, JitScale jit) {
-    q2d_kernel_body<InT, FMT, COLSUM, true, false, false, true>(x, rows, cols, cols, vec_ok, nullptr, q, ldq, qt,
-                                                                ldqt, colpart, nullptr, LnArgs(), jit);
-}
-
+// The just-in-time pass (df_quantize_2d_jit), x contiguous, held to five
+// waves per SIMD, the occupancy of the same pass without the fold (the fold's
+// registers are dead before the tile pass).  COLSUM: finishes the column sums.
 template <typename InT, int FMT, bool COLSUM>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) void quantize_2d_jit_w5_kernel(
     const InT* __restrict__ x, int rows, int cols, bool vec_ok, uint8_t* __restrict__ q, int ldq,
-    uint8_t* __restrict__ qt, int ldqt, float* __restrict__ colpart, JitScale jit) {
+    uint8_t* __restrict__ qt, int ldqt, JitScale jit) {
     q2d_kernel_body<InT, FMT, COLSUM, true, false, false, true>(x, rows, cols, cols, vec_ok, nullptr, q, ldq, qt,
-                                                                ldqt, colpart, nullptr, LnArgs(), jit);
+                                                                ldqt, nullptr, nullptr, LnArgs(), jit);
 }
 
+// The same in one launch for a small x.
 template <typename InT, int FMT, bool COLSUM>
 __global__ __launch_bounds__(kThreads) void quantize_2d_jit_scan_kernel(const InT* __restrict__ x, int rows, int cols,
                                                                          bool vec_ok, uint8_t* __restrict__ q, int ldq,
@@ -1083,12 +1210,9 @@ static void launch_q2d_jit(dim3 grid, hipStream_t st, const InT* x, int rows, in
     if (!jit.nparts)
         quantize_2d_jit_scan_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
                                                                                   ldqt, colpart, jit);
-    else if constexpr (sizeof(InT) == 2 || !COLSUM)
-        quantize_2d_jit_w5_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
-                                                                                ldqt, colpart, jit);
     else
-        quantize_2d_jit_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt, ldqt,
-                                                                             colpart, jit);
+        quantize_2d_jit_w5_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
+                                                                                ldqt, jit);
 }
 
 // ---- several 2-D tensors in two launches (every Linear's weights after an
@@ -1610,15 +1734,36 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
         return DF_OK;
     }
     DF_CHECK(grid.y <= 65535, DF_ERR_INVALID, "%s: rows=%d too large", name, rows);
-    float* part = colsum ? static_cast<float*>(ws) : nullptr;
+    // one row of tiles: its sums are the column sums, nothing to reduce
+    const int tile_rows = (rows + kT2R - 1) / kT2R;
+    float* part = !colsum ? nullptr : tile_rows == 1 ? colsum : static_cast<float*>(ws);
+    bool reduce = colsum && tile_rows != 1;
     uint32_t* amaxpart = delayed ? reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + amax_off) : nullptr;
     const int esz = in_dtype == DF_DTYPE_FLOAT32 ? 4 : 2;
     const bool vec_ok = aligned16(x) && ((int64_t)ldx * esz) % 16 == 0;
     JitScale J;
     if (jit) {
         uint32_t* jparts = reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + jit_off);
-        if ((int64_t)rows * cols * esz > kJitScanBytes)
-            J.nparts = launch_absmax_stage1(in_dtype, x, (int64_t)rows * cols, jparts, st, kJitParts);
+        if ((int64_t)rows * cols * esz > kJitScanBytes) {
+            if (colsum) {
+                J.nparts = (int)std::min<int64_t>(kJitParts, (int64_t)tile_rows * ((cols + kT2 - 1) / kT2));
+#define DF_ACS(T)                                                                                             \
+    absmax_colsum_stage1<T><<<J.nparts, kThreads, 0, st>>>(static_cast<const T*>(x), rows, cols, vec_ok,      \
+                                                           jparts, part)
+                if (in_dtype == DF_DTYPE_FLOAT32) DF_ACS(float);
+                else if (in_dtype == DF_DTYPE_HALF) DF_ACS(f16_t);
+                else DF_ACS(uint16_t);
+#undef DF_ACS
+                if (reduce) {  // by the first row of tile blocks
+                    J.colpart = part;
+                    J.colsum = colsum;
+                    J.tile_rows = tile_rows;
+                    reduce = false;
+                }
+            } else {
+                J.nparts = launch_absmax_stage1(in_dtype, x, (int64_t)rows * cols, jparts, st, kJitParts);
+            }
+        }
         J.parts = jparts;
         J.absmax_out = jit_absmax;
         J.scale_out = const_cast<float*>(scale_dev);
@@ -1656,9 +1801,7 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
         else { if (colsum) DF_Q2D(uint16_t, E5M2, true); else DF_Q2D(uint16_t, E5M2, false); }
     }
 #undef DF_Q2D
-    if (colsum)
-        colsum_reduce_kernel<<<(cols + 63) / 64, kThreads, 0, st>>>(part, rows == 0 ? 0 : (rows + kT2R - 1) / kT2R,
-                                                                    cols, colsum);
+    if (reduce) colsum_reduce_kernel<<<(cols + 63) / 64, kThreads, 0, st>>>(part, tile_rows, cols, colsum);
     if (delayed)
         amax_history_kernel<<<1, kThreads, 0, st>>>(amaxpart, (int)(grid.x * grid.y), fmt, history, hist_len,
                                                     next_scale);
