@@ -66,3 +66,41 @@ def test_edges(dev, rows, cols, dt, fmt):
     wide = torch.full((rows, cols + 3), float("nan"), dtype=dt, device=dev)
     wide[:, :cols].copy_(x)
     check(*df.quantize_2d(wide[:, :cols], sc, fmt, want_qt=True))
+
+
+# rows of whole 16-byte chunks below, at and past what a wave's registers hold,
+# row counts that leave waves with fewer rows than their share, rows too wide
+# for the registers in whole and part rounds of sixteen values a lane
+@pytest.mark.parametrize("rows,cols", [(1, 8), (5, 512), (130, 1600), (67, 2048), (9, 1024), (8193, 64), (16387, 72),
+                                       (6, 2056), (3, 6400), (4, 3001)])
+@pytest.mark.parametrize("dt", [F32, BF16, F16])
+@pytest.mark.parametrize("affine", [True, False])
+def test_layernorm_codes(dev, rows, cols, dt, affine):
+    """The fused LayerNorm's codes and scale are those of the quantize of its
+    own y, and y is within rounding of binary64 (a NaN row, a constant row and
+    values that overflow the element type among them)."""
+    g = torch.Generator().manual_seed(rows + 31 * cols)
+    x = torch.randn(rows, cols, generator=g) * 2 + 0.25
+    if rows > 4:
+        x[1, cols // 2] = float("nan")
+        x[2] = 0.5
+    x = x.to(dt).to(dev)
+    gamma = (1 + 0.1 * torch.randn(cols, generator=g)).to(dt).to(dev) if affine else None
+    beta = (0.1 * torch.randn(cols, generator=g)).to(dt).to(dev) if affine else None
+    y0 = df.layernorm(x, gamma, beta)
+    y, q, qt, sc = df.layernorm(x, gamma, beta, fmt=Fmt.E4M3, want_y=True, want_qt=True)
+    bits = torch.int32 if dt == F32 else torch.int16
+    assert torch.equal(y.view(bits), y0.view(bits))
+    _, sy, q2, qt2 = df.quantize_2d_jit(y.contiguous(), Fmt.E4M3, want_qt=True)
+    assert sc.item() == sy.item() and torch.equal(q, q2) and torch.equal(qt, qt2)
+    xd = x.double()
+    ref = (xd - xd.mean(1, keepdim=True)) / (xd.var(1, unbiased=False, keepdim=True) + 1e-5).sqrt()
+    if affine:
+        ref = ref * gamma.double() + beta.double()
+    ok = torch.isfinite(ref)
+    # half a unit in the last place of a p-bit significand is at most 2^-p of the value (p = 24, 8, 11); behind it
+    # binary32 sums of `cols` values of magnitude below 8
+    ulp = {F32: 2.0 ** -24, BF16: 2.0 ** -8, F16: 2.0 ** -11}[dt]
+    err = (y.double() - ref).abs()[ok]
+    bound = ulp * ref.abs()[ok] + cols * 2.0 ** -24 * 8 + 2.0 ** -25
+    assert bool((err <= bound).all()) and bool(torch.isnan(y[~ok]).all())
