@@ -24,13 +24,13 @@ constexpr int kMaxReduceBlocks = 2048;  // partials in the absmax workspace
 // partials, so fewer than kMaxReduceBlocks (512: 2 KiB per tile block, and
 // still enough blocks for the absmax pass to stream at full rate)
 constexpr int kJitParts = 512;
-// df_quantize_2d_jit inputs of at most this many bytes run in one launch: each
-// tile block reads all of x for the absmax (one chunk of kU loads per thread)
-// instead of folding the partials of a pass before it.  8 x 1600 bf16 (25 KB):
-// 6.3 us against 8.4 with the separate pass; beyond one chunk the blocks' scans
-// cost what the launch saves (40 x 1000, 80 KB: 8.5 against 9.0; 8 x 6400,
-// 102 KB: 8.8 against 8.5; 64 x 1600, 205 KB: 11.3 against 8.5).
-constexpr int64_t kJitScanBytes = 32 << 10;
+// df_quantize_2d_jit inputs of at most this many bytes (no column sums) run in
+// one launch: each tile block reads all of x for the absmax (32 KB a round of
+// kU loads per thread) instead of folding the partials of a pass before it.
+// One launch against two, us: 8 x 4096 bf16 (64 KB) 5.0 / 6.8, 40 x 1000
+// (80 KB) 6.2 / 7.9, 8 x 6400 (100 KB) 5.9 / 6.7; a further round costs what
+// is left of the gain.
+constexpr int64_t kJitScanBytes = 128 << 10;
 
 // plain or non-temporal (NT) accesses.  The flat kernels store
 // non-temporal (NTS) when their output starts on a 128-byte boundary: every
@@ -85,20 +85,9 @@ constexpr int kUQuantF32 = 2, kUQuantBf16 = 4, kUDeqF32 = 2, kUDeqBf16 = 1;
 // Stage 1 body: the block's maximum over its chunks (block bi of nb blocks
 // walking the chunks with a stride of nb).  |x| bit patterns, NaN and
 // infinities skipped (fold_*).  InT: float, uint16_t (bf16) or f16_t.
-__device__ __forceinline__ uint32_t fold_f16x2(uint32_t m, uint32_t w) {
-    m = fold_f32(m, __float_as_uint(f16_to_f32(w & 0xFFFFu)));
-    return fold_f32(m, __float_as_uint(f16_to_f32(w >> 16)));
-}
-template <typename InT> __device__ __forceinline__ uint32_t fold_vec(uint32_t m, const u32x4 v) {
-    if constexpr (std::is_same<InT, float>::value) {
-        m = fold_f32(m, v.x); m = fold_f32(m, v.y); m = fold_f32(m, v.z); return fold_f32(m, v.w);
-    } else if constexpr (std::is_same<InT, f16_t>::value) {
-        m = fold_f16x2(m, v.x); m = fold_f16x2(m, v.y); m = fold_f16x2(m, v.z); return fold_f16x2(m, v.w);
-    } else {
-        m = fold_bf16x2(m, v.x); m = fold_bf16x2(m, v.y); m = fold_bf16x2(m, v.z); return fold_bf16x2(m, v.w);
-    }
-}
-// the compare-free forms (df_common.hpp): three operations per dword
+// The folds are the compare-free forms (df_common.hpp): three operations per
+// dword against six to twelve, and a fifth of the f16 pass's code, which is what
+// a pass over a small input waits for (16384 x 6400 bf16: 34.9 us against 36.2).
 template <typename InT> __device__ __forceinline__ uint32_t fold_vec_biased(uint32_t m, const u32x4 v) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -113,10 +102,10 @@ template <typename InT> __device__ __forceinline__ uint32_t unbias(uint32_t m) {
     else if constexpr (std::is_same<InT, f16_t>::value) return unbias_f16x2(m);
     else return unbias_bf16x2(m);
 }
-template <typename InT> __device__ __forceinline__ uint32_t fold_one(uint32_t m, const InT* p) {
-    if constexpr (std::is_same<InT, float>::value) return fold_f32(m, __float_as_uint(*p));
-    else if constexpr (std::is_same<InT, f16_t>::value) return fold_f32(m, __float_as_uint(f16_to_f32(p->bits)));
-    else return fold_f32(m, (uint32_t)*p << 16);
+template <typename InT> __device__ __forceinline__ uint32_t fold_one_biased(uint32_t m, const InT* p) {
+    if constexpr (std::is_same<InT, float>::value) return fold_f32_biased(m, __float_as_uint(*p));
+    else if constexpr (std::is_same<InT, f16_t>::value) return fold_f16x2_biased(m, p->bits);
+    else return fold_bf16x2_biased(m, *p);
 }
 
 template <typename InT, bool NT = true>
@@ -132,7 +121,7 @@ __device__ __forceinline__ uint32_t absmax_block(const InT* __restrict__ x, int6
         for (int u = 0; u < kU; ++u) v[u] = ld_nt<NT>(xv + base + u * kThreads + threadIdx.x);
         __builtin_amdgcn_sched_barrier(0);  // no fold before the last load has left
 #pragma unroll
-        for (int u = 0; u < kU; ++u) m = fold_vec<InT>(m, v[u]);
+        for (int u = 0; u < kU; ++u) m = fold_vec_biased<InT>(m, v[u]);
     }
     if (base < nvec) {
         // the last, partial chunk: loads past it take the last vector again
@@ -141,10 +130,10 @@ __device__ __forceinline__ uint32_t absmax_block(const InT* __restrict__ x, int6
 #pragma unroll
         for (int u = 0; u < kU; ++u) v[u] = xv[min(base + u * kThreads + (int64_t)threadIdx.x, nvec - 1)];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) m = fold_vec<InT>(m, v[u]);
+        for (int u = 0; u < kU; ++u) m = fold_vec_biased<InT>(m, v[u]);
     }
-    if (bi == 0 && threadIdx.x < n - nvec * E) m = fold_one<InT>(m, x + nvec * E + threadIdx.x);
-    return block_max_u32(m);
+    if (bi == 0 && threadIdx.x < n - nvec * E) m = fold_one_biased<InT>(m, x + nvec * E + threadIdx.x);
+    return block_max_u32(unbias<InT>(m));
 }
 
 // Stage 1: one partial maximum per block.
@@ -1289,8 +1278,7 @@ __device__ __forceinline__ void finish_colsum(const float* __restrict__ colpart,
 
 // JIT: the scale comes from the absmax partials in jit (jit_block_scale;
 // block (0, 0) writes absmax and scale), not from scale[0].
-// SCAN: a small x, whose absmax every block takes itself (kJitScanBytes).
-template <typename InT, int FMT, bool COLSUM, bool CODES, bool AMAX, bool LN, bool JIT, bool SCAN = false>
+template <typename InT, int FMT, bool COLSUM, bool CODES, bool AMAX, bool LN, bool JIT>
 __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int rows, int cols, int ldx, bool vec_ok,
                                                 const float* __restrict__ scale, uint8_t* __restrict__ q, int ldq,
                                                 uint8_t* __restrict__ qt, int ldqt, float* __restrict__ colpart,
@@ -1299,17 +1287,13 @@ __device__ __forceinline__ void q2d_kernel_body(const InT* __restrict__ x, int r
     static_assert(!JIT || (CODES && !AMAX && !LN), "just-in-time scale: the plain code pass");
     constexpr int RG = kThreads / (kT2 / Ld<InT>::E);
     __shared__ __attribute__((aligned(16))) uint8_t tile[kT2 * kT2R];
-    // a two-pass just-in-time call has its sums from the absmax pass
-    constexpr bool TILE_SUMS = COLSUM && !(JIT && !SCAN);
+    // a just-in-time call has its sums from the absmax pass
+    constexpr bool TILE_SUMS = COLSUM && !JIT;
     __shared__ float csum[TILE_SUMS ? RG : 1][kT2];
     float sc = 1.0f;
     if constexpr (JIT) {
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-        if constexpr (SCAN)
-            sc = block_scale(absmax_block<InT, false>(x, (int64_t)rows * cols, 0, 1), FMT, jit.absmax_out,
-                             jit.scale_out, writer);
-        else
-            sc = jit_block_scale(jit.parts, jit.nparts, FMT, jit.absmax_out, jit.scale_out, writer);
+        sc = jit_block_scale(jit.parts, jit.nparts, FMT, jit.absmax_out, jit.scale_out, writer);
     }
     if constexpr (CODES && !JIT) sc = scale[0];
     const QDiv d = make_qdiv(sc);
@@ -1357,22 +1341,125 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
                                                                 ldqt, nullptr, nullptr, LnArgs(), jit);
 }
 
-// The same in one launch for a small x.
-template <typename InT, int FMT, bool COLSUM>
-__global__ __launch_bounds__(kThreads) void quantize_2d_jit_scan_kernel(const InT* __restrict__ x, int rows, int cols,
-                                                                         bool vec_ok, uint8_t* __restrict__ q, int ldq,
-                                                                         uint8_t* __restrict__ qt, int ldqt,
-                                                                         float* __restrict__ colpart, JitScale jit) {
-    q2d_kernel_body<InT, FMT, COLSUM, true, false, false, true, true>(x, rows, cols, cols, vec_ok, nullptr, q, ldq, qt,
-                                                                      ldqt, colpart, nullptr, LnArgs(), jit);
+// Tile grid of a 2-D quantize (tiles of tr rows and kT2 columns): covers the
+// codes' padded extents.
+static dim3 q2d_grid(int rows, int cols, const uint8_t* q, int ldq, const uint8_t* qt, int ldqt, int tr) {
+    const int row_ext = qt ? (rows > ldqt ? rows : ldqt) : rows;
+    const int col_ext = q ? (cols > ldq ? cols : ldq) : cols;
+    return dim3((col_ext + kT2 - 1) / kT2, (row_ext + tr - 1) / tr);
+}
+
+// The just-in-time pass over few tiles (kSmallTiles).  Such a launch is a
+// chain of latencies: fetching the kernel's code, the absmax partials, x, a
+// thread's conversions one after the other.  quantize_2d_jit_w5_kernel is
+// built for throughput (58-81 KB of code, 64 values a thread); this one is
+// built for the chain: a thread has four rows of 16 bytes, its loads leave
+// before the partials are folded, and the conversion that every value can take
+// (IEEE division, NaN) stands apart from the one that nearly all take.  Codes,
+// scale and sums are the same bit for bit.  A call takes (us, against the
+// throughput kernel): 8 x 1600 bf16 4.6 (6.6), 64 x 768 fp32 6.3 (9.3),
+// 512 x 768 with both codes 7.9 (8.5), 1000 x 771 f16 9.4 (15.0).
+// SCAN: the absmax is taken here, not folded (kJitScanBytes).
+template <typename InT, int FMT, bool SCAN>
+__global__ __launch_bounds__(kThreads) void quantize_2d_small_kernel(const InT* __restrict__ x, int rows, int cols,
+                                                                      uint8_t* __restrict__ q, int ldq,
+                                                                      uint8_t* __restrict__ qt, int ldqt,
+                                                                      JitScale jit) {
+    constexpr int E = Ld<InT>::E, TPR = kT2 / E, RG = kThreads / TPR, RPT = 4, TR = RG * RPT;
+    constexpr int LS = TR + 16;  // a transposed column in LDS
+    __shared__ __attribute__((aligned(16))) uint8_t tile[kT2 * LS];
+    const int c0 = blockIdx.x * kT2, r0 = blockIdx.y * TR;
+    const int tc = (threadIdx.x % TPR) * E, rg = threadIdx.x / TPR, c = c0 + tc, r1 = r0 + rg * RPT;
+    // a chunk that runs past the row's end is read as the row's last E
+    // values; `by` bytes of it lie before column c
+    const int over = c + E - cols, cl = over > 0 ? cols - E : c;
+    u32x4 raw[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+        raw[i] = u32x4{0, 0, 0, 0};
+        if (r1 + i < rows && c < cols)
+            raw[i] = cols >= E ? ld16_any(x + (int64_t)(r1 + i) * cols + cl)
+                               : ld_short<InT>(x + (int64_t)(r1 + i) * cols, c, cols);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
+    float sc;
+    if constexpr (SCAN)
+        sc = block_scale(absmax_block<InT, false>(x, (int64_t)rows * cols, 0, 1), FMT, jit.absmax_out, jit.scale_out,
+                         writer);
+    else
+        sc = jit_block_scale(jit.parts, jit.nparts, FMT, jit.absmax_out, jit.scale_out, writer);
+    const QDiv d = make_qdiv(sc);
+    const int by = over > 0 && c < cols && cols >= E ? over * (int)sizeof(InT) : 0;
+    float v[RPT * E];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) Ld<InT>::widen(drop_bytes(raw[i], by), v + i * E);
+    uint32_t codes[RPT][E / 4];
+    if (__builtin_expect(d.fast && !wave_any_nan<RPT * E>(v), 1)) {
+#pragma unroll
+        for (int k = 0; k < RPT * E / 4; ++k)
+            codes[k / (E / 4)][k % (E / 4)] = quant4_nonan<FMT>(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3], d);
+    } else {
+#pragma unroll
+        for (int k = 0; k < RPT * E / 4; ++k)
+            codes[k / (E / 4)][k % (E / 4)] =
+                quant4_t<FMT, false>(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3], d);
+    }
+    if (q && c < ldq) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            uint8_t* const dst = q + (int64_t)(r1 + i) * ldq + c;
+            if (r1 + i < rows) {
+                if (E == 8) *reinterpret_cast<u32x2*>(dst) = u32x2{codes[i][0], codes[i][E / 4 - 1]};
+                else *reinterpret_cast<uint32_t*>(dst) = codes[i][0];
+            }
+        }
+    }
+    if (qt) {
+#pragma unroll
+        for (int g = 0; g < E / 4; ++g) {
+            uint32_t col[4];
+            transpose4x4_bytes(codes[0][g], codes[1][g], codes[2][g], codes[3][g], col);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *reinterpret_cast<uint32_t*>(tile + (tc + 4 * g + j) * LS + rg * RPT) = col[j];
+        }
+        __syncthreads();
+        constexpr int CPC = TR / 16;  // 16-byte chunks per column
+#pragma unroll
+        for (int k = 0; k < kT2 * CPC / kThreads; ++k) {
+            const int idx = threadIdx.x + kThreads * k, tcol = idx / CPC, rc = (idx % CPC) * 16;
+            if (c0 + tcol < cols && r0 + rc < ldqt)
+                *reinterpret_cast<u32x4*>(qt + (int64_t)(c0 + tcol) * ldqt + r0 + rc) =
+                    *reinterpret_cast<const u32x4*>(tile + tcol * LS + rc);
+        }
+    }
+    if constexpr (!SCAN) {
+        if (blockIdx.y == 0 && jit.colsum)
+            finish_colsum(jit.colpart, jit.tile_rows, cols, c0, jit.colsum);
+    }
+}
+
+// 128x128 tiles up to which the small kernel runs: one per CU.  At 384 tiles
+// (8192 x 768) the two kernels are even (14.2 us), at 1664 (16384 x 1600) it is
+// 35.5 against 32.5 us.
+constexpr int kSmallTiles = 256;
+
+template <typename InT, int FMT>
+static void launch_q2d_small(hipStream_t st, const InT* x, int rows, int cols, uint8_t* q, int ldq, uint8_t* qt,
+                             int ldqt, const JitScale& jit) {
+    const dim3 grid = q2d_grid(rows, cols, q, ldq, qt, ldqt, 4 * (kThreads / (kT2 / Ld<InT>::E)));
+    if (jit.nparts)
+        quantize_2d_small_kernel<InT, FMT, false><<<grid, kThreads, 0, st>>>(x, rows, cols, q, ldq, qt, ldqt, jit);
+    else
+        quantize_2d_small_kernel<InT, FMT, true><<<grid, kThreads, 0, st>>>(x, rows, cols, q, ldq, qt, ldqt, jit);
 }
 
 template <typename InT, int FMT, bool COLSUM>
 static void launch_q2d_jit(dim3 grid, hipStream_t st, const InT* x, int rows, int cols, bool vec_ok, uint8_t* q,
-                           int ldq, uint8_t* qt, int ldqt, float* colpart, const JitScale& jit) {
-    if (!jit.nparts)
-        quantize_2d_jit_scan_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
-                                                                                  ldqt, colpart, jit);
+                           int ldq, uint8_t* qt, int ldqt, const JitScale& jit) {
+    if (!jit.nparts || (int64_t)grid.x * grid.y <= kSmallTiles)
+        launch_q2d_small<InT, FMT>(st, x, rows, cols, q, ldq, qt, ldqt, jit);
     else
         quantize_2d_jit_w5_kernel<InT, FMT, COLSUM><<<grid, kThreads, 0, st>>>(x, rows, cols, vec_ok, q, ldq, qt,
                                                                                 ldqt, jit);
@@ -1816,14 +1903,6 @@ extern "C" size_t df_quantize_2d_jit_workspace_bytes(int rows, int cols, int col
     return jit_ws_layout(rows, cols, colsum != 0, nullptr);
 }
 
-// Tile grid of a 2-D quantize (tiles of tr rows and kT2 columns): covers the
-// codes' padded extents.
-static dim3 q2d_grid(int rows, int cols, const uint8_t* q, int ldq, const uint8_t* qt, int ldqt, int tr) {
-    const int row_ext = qt ? (rows > ldqt ? rows : ldqt) : rows;
-    const int col_ext = q ? (cols > ldq ? cols : ldq) : cols;
-    return dim3((col_ext + kT2 - 1) / kT2, (row_ext + tr - 1) / tr);
-}
-
 // Delayed-scaling workspace: column-sum partials (when asked for), then one
 // tile maximum per block, 16-byte aligned.
 static size_t delayed_ws_layout(int rows, int cols, int ldq, int ldqt, bool colsum, size_t* amax_off) {
@@ -1907,7 +1986,8 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
     JitScale J;
     if (jit) {
         uint32_t* jparts = reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + jit_off);
-        if ((int64_t)rows * cols * esz > kJitScanBytes) {
+        const int64_t n = (int64_t)rows * cols;
+        if (n > 0 && (colsum || n * esz > kJitScanBytes)) {
             if (colsum) {
                 J.nparts = (int)std::min<int64_t>(kJitParts, (int64_t)tile_rows * ((cols + kT2 - 1) / kT2));
 #define DF_ACS(T)                                                                                             \
@@ -1924,7 +2004,7 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
                     reduce = false;
                 }
             } else {
-                J.nparts = launch_absmax_stage1(in_dtype, x, (int64_t)rows * cols, jparts, st, kJitParts);
+                J.nparts = launch_absmax_stage1(in_dtype, x, n, jparts, st, kJitParts);
             }
         }
         J.parts = jparts;
@@ -1934,8 +2014,7 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
 #define DF_Q2D(T, F, CS)                                                                                        \
     do {                                                                                                        \
         if (jit)                                                                                                \
-            launch_q2d_jit<T, F, CS>(grid, st, static_cast<const T*>(x), rows, cols, vec_ok, q, ldq, qt, ldqt,   \
-                                     part, J);                                                                  \
+            launch_q2d_jit<T, F, CS>(grid, st, static_cast<const T*>(x), rows, cols, vec_ok, q, ldq, qt, ldqt, J); \
         else if (delayed)                                                                                       \
             quantize_2d_kernel<T, F, CS, true, true><<<grid, kThreads, 0, st>>>(                                \
                 static_cast<const T*>(x), rows, cols, ldx, vec_ok, scale_dev, q, ldq, qt, ldqt, part, amaxpart); \

@@ -15,9 +15,11 @@ pytestmark = pytest.mark.gpu
 
 F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
 # one value, rows shorter than a 16-byte chunk, one value past / short of a
-# chunk and of a tile, 32 KB of input on, below and above (the one-launch form's limit)
+# chunk and of a tile, 128 KB of input on, below and above (the one-launch form's limit in 2 and 4 byte types),
+# tiles on and past the small kernel's limit
 SHAPES = [(1, 1), (3, 3), (5, 7), (129, 5), (2, 9), (127, 129), (128, 127), (130, 136), (257, 131), (8, 1600),
-          (16, 1024), (16, 1025), (31, 264), (64, 128), (8, 1023), (300, 77)]
+          (16, 1024), (16, 1025), (31, 264), (64, 128), (8, 1023), (300, 77),
+          (64, 1024), (64, 1025), (32, 1024), (33, 1024), (2048, 2048), (2049, 2056)]
 
 
 def tensor(rows, cols, dt, dev, seed):
