@@ -542,7 +542,7 @@ EXTRA_STATS = (
      ("adam_kernel", "sumsq_kernel", "clip_kernel", "norm_finalize_kernel")),
     ("stats_producer", "prof_producer", "layernorm_quantize_kernel_stats.md",
      "LayerNorm + e4m3 codes, 16384 x 1600 bf16 (unfused chain, fused, fused delayed)",
-     ("ln_stats_kernel", "true>(unsigned short const*", "amax_history_kernel")),
+     ("ln_stats_", "true>(unsigned short const*", "true, false>(unsigned short const*", "amax_history_kernel")),
     ("stats_producer", "prof_producer", "gemm_producer_kernel_stats.md",
      "GEMMs that also fold their output's absmax: fc1's forward and fc2's grouped backward at the config-4 fc "
      "shapes (the producer leg's gemm_producer variants)",
