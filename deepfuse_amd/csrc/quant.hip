@@ -1989,7 +1989,9 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
     if (jit) {
         uint32_t* jparts = reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + jit_off);
         const int64_t n = (int64_t)rows * cols;
-        if (n > 0 && (colsum || n * esz > kJitScanBytes)) {
+        // one launch: a small x, and few tiles (each reads all of x)
+        const bool scan = !colsum && n * esz <= kJitScanBytes && (int64_t)grid.x * grid.y <= kSmallTiles;
+        if (n > 0 && !scan) {
             if (colsum) {
                 J.nparts = (int)std::min<int64_t>(kJitParts, (int64_t)tile_rows * ((cols + kT2 - 1) / kT2));
 #define DF_ACS(T)                                                                                             \

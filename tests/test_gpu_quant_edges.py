@@ -19,7 +19,8 @@ F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
 # tiles on and past the small kernel's limit
 SHAPES = [(1, 1), (3, 3), (5, 7), (129, 5), (2, 9), (127, 129), (128, 127), (130, 136), (257, 131), (8, 1600),
           (16, 1024), (16, 1025), (31, 264), (64, 128), (8, 1023), (300, 77),
-          (64, 1024), (64, 1025), (32, 1024), (33, 1024), (2048, 2048), (2049, 2056)]
+          (64, 1024), (64, 1025), (32, 1024), (33, 1024), (2048, 2048), (2049, 2056),
+          (40000, 1)]
 
 
 def tensor(rows, cols, dt, dev, seed):
