@@ -1155,6 +1155,38 @@ __global__ __launch_bounds__(kThreads) void ln_stats_whole_kernel(const InT* __r
     }
 }
 
+// A long list of partials (16-byte aligned, `out` behind it) down to kFewParts,
+// one per block, for a pass whose every block folds what it is given.  Eight
+// 16-byte loads in flight per thread: 32768 partials are one round.
+constexpr int kFewParts = 4;
+// LayerNorm to codes: partials up to which every tile block folds all of them
+// (32 KB).  More are first folded to kFewParts, since the blocks' reads grow
+// with the square of the rows; the statistics pass itself is not held to fewer
+// blocks, whose loop over rows costs it its occupancy (131072 x 1601 bf16: 941
+// to 1174 us a call with 2048 to 512 partials against 756).  A call takes (us,
+// bf16 and f16, every block folding all / folded first): 4096 partials, 16384 x
+// 129, 24.9 / 26.6; 8192, 32768 x 65, 36.6 / 37.5; 16384, 65536 x 33, 39.3 /
+// 38.9; 32768, 131072 x 1601, 756 / 746; 262144, 1048576 x 65, 848 / 637.
+constexpr int kLnFoldParts = 8192;
+__global__ __launch_bounds__(kThreads) void fold_to_few_kernel(const uint32_t* __restrict__ part, int nparts,
+                                                               uint32_t* __restrict__ out) {
+    constexpr int S = kFewParts * kThreads;
+    const u32x4* p = reinterpret_cast<const u32x4*>(part);
+    const int n4 = nparts >> 2;
+    u32x4 m{0, 0, 0, 0};
+    for (int i = blockIdx.x * kThreads + threadIdx.x; i < n4; i += 8 * S) {
+        u32x4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[min(i + u * S, n4 - 1)];  // past the end: the last one again
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m = __builtin_elementwise_max(m, v[u]);
+    }
+    uint32_t r = max(max(m.x, m.y), max(m.z, m.w));
+    if (blockIdx.x == 0 && threadIdx.x < (nparts & 3)) r = max(r, part[4 * n4 + threadIdx.x]);
+    r = block_max_u32(r);
+    if (threadIdx.x == 0) out[blockIdx.x] = r;
+}
+
 // history[0..len) = amax (or 0 when amax is NULL), scale from it.
 __global__ __launch_bounds__(kThreads) void amax_history_init_kernel(const float* __restrict__ amax, int fmt,
                                                                       float* __restrict__ history, int len,
@@ -2312,14 +2344,15 @@ extern "C" int df_quantize_2d_batch_absmax(int in_dtype, int count, const void* 
 
 // ---------------------------------------------------------------- LayerNorm --
 // Workspace: (mean, rstd) per row, then the absmax partials of the
-// statistics pass or of the tile pass (delayed), 16-byte aligned.
+// statistics pass or of the tile pass (delayed), 16-byte aligned, and behind
+// them room for kFewParts more.
 static size_t ln_ws_layout(int rows, int cols, int ldq, int ldqt, size_t* part_off) {
     const size_t st = ((size_t)rows * sizeof(float2) + 15) & ~(size_t)15;
     const size_t stat_parts = (size_t)((rows + 3) / 4);
     const dim3 g = q2d_grid(rows, cols, (const uint8_t*)1, ldq, ldqt > 0 ? (const uint8_t*)1 : nullptr, ldqt, kT2R);
     const size_t tile_parts = (size_t)g.x * g.y;
     if (part_off) *part_off = st;
-    return st + (stat_parts > tile_parts ? stat_parts : tile_parts) * sizeof(uint32_t) + 16;
+    return st + (stat_parts > tile_parts ? stat_parts : tile_parts) * sizeof(uint32_t) + kFewParts * sizeof(uint32_t);
 }
 
 extern "C" size_t df_layernorm_workspace_bytes(int rows, int cols, int ldq, int ldqt) {
@@ -2398,9 +2431,9 @@ static int layernorm_impl(const char* name, int mode, int dtype, const void* x, 
     const int esz = (bf || h16) ? 2 : 4;
     const bool vec_ok = aligned16(x) && ((int64_t)ldx * esz) % 16 == 0;
     const bool gb_vec = gamma && aligned16(gamma) && aligned16(beta);
-    // rows per wave of the whole-chunk kernel: as many as leave two to four
-    // blocks per CU (every tile block of the just-in-time form folds the
-    // blocks' partials)
+    // rows per wave of the whole-chunk kernel: one up to 4095 rows, then as many
+    // as leave two to four blocks per CU (512 to 1024 partials), at most eight
+    // (32768 rows and more: a partial per 32 rows)
     const int chunk = 16 / esz, rpw = std::min(8, std::max(1, rows / 2048));
     const bool whole = vec_ok && cols % chunk == 0 && cols <= 64 * chunk * kLnRegChunks;
     if (whole) sblocks = (sblocks + rpw - 1) / rpw;
@@ -2418,11 +2451,16 @@ static int layernorm_impl(const char* name, int mode, int dtype, const void* x, 
     DF_BY_TYPE(if (mode == 1) DF_LNS(T, true); else DF_LNS(T, false));
 #undef DF_LNS
     // tile pass; just in time, its blocks fold the statistics pass's partials
-    // (16384 x 1600 bf16: 37.9 us a call against 40.1 with a launch for the
-    // fold, 64 x 768: 12.4 against 13.6)
+    // (16384 x 1600 bf16: 37.9 us a call against 40.1 with a launch that folds
+    // them to the scale, 64 x 768: 12.4 against 13.6), long lists folded first
     JitScale J;
     J.parts = parts;
     J.nparts = sblocks;
+    if (mode == 1 && sblocks > kLnFoldParts) {  // the layout has room for kFewParts behind them
+        fold_to_few_kernel<<<kFewParts, kThreads, 0, st>>>(parts, sblocks, parts + sblocks);
+        J.parts = parts + sblocks;
+        J.nparts = kFewParts;
+    }
     J.absmax_out = next_scale;
     J.scale_out = const_cast<float*>(scale_dev);
     LnArgs la;

@@ -107,3 +107,37 @@ def test_layernorm_codes(dev, rows, cols, dt, affine):
     err = (y.double() - ref).abs()[ok]
     bound = ulp * ref.abs()[ok] + cols * 2.0 ** -24 * 8 + 2.0 ** -25
     assert bool((err <= bound).all()) and bool(torch.isnan(y[~ok]).all())
+
+
+# one and three partials past the count (8192) up to which every tile block of
+# the fused LayerNorm folds them all: rows of odd width have a partial per 4
+# rows, rows of whole 16-byte chunks one per 32
+@pytest.mark.parametrize("rows,cols,per", [(32772, 33, 4), (32777, 5, 4), (262176, 64, 32)])
+@pytest.mark.parametrize("at", ["first", "middle", "last"])
+def test_layernorm_many_rows(dev, rows, cols, per, at):
+    """A long list of absmax partials is folded before the tile pass, whose
+    every block would otherwise read all of it: the folded values lie behind
+    the list in the workspace, and codes, scale and absmax are those of the
+    quantize of y wherever the largest |y| stands."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=g).clamp_(-2, 2)
+    r = {"first": 0, "middle": rows // 2, "last": rows - 1}[at]
+    x[r] = 0.0
+    x[r, cols // 2] = 100.0  # a one-hot row has the largest normalized value of all
+    x = x.to(BF16).to(dev)
+    y = df.layernorm(x)
+    am, sy, q2, qt2 = df.quantize_2d_jit(y, Fmt.E4M3, want_qt=True)
+    q, qt = torch.empty_like(q2), torch.empty_like(qt2)
+    sc, ab = torch.empty(1, device=dev), torch.empty(1, device=dev)
+    nbytes = df.lib().df_layernorm_workspace_bytes(rows, cols, q.shape[1], qt.shape[1])
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev)
+    df.call("df_layernorm_quantize", int(df.DType.BFLOAT16), x.data_ptr(), rows, cols, cols, None, None, 1e-5, None, 0,
+            int(Fmt.E4M3), sc.data_ptr(), ab.data_ptr(), q.data_ptr(), q.shape[1], qt.data_ptr(), qt.shape[1],
+            ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    assert sc.item() == sy.item() and ab.item() == am.item() == y[r].float().abs().max().item()
+    assert torch.equal(q, q2) and torch.equal(qt, qt2)
+    parts = ws[(rows * 8 + 15) // 16 * 16:].view(torch.float32)
+    n = (rows + per - 1) // per
+    few = parts[n:n + 4]
+    assert n > 8192 and bool(torch.isfinite(parts[:n + 4]).all())
+    assert parts[:n].max().item() == few.max().item() == am.item()
