@@ -1278,6 +1278,13 @@ static void launch_persistent_narrow(const GemmArgs& g, int grid) {
 // faster there), while the GPT-2 XL shapes at 16384 tokens keep 256x256
 // tiles (narrow ones 13-40% slower).
 constexpr double kNarrowStep = 0.6, kNarrowOverhead = 2.0;
+// The same two as measured, for a price that is compared with other launches'
+// (grouped_plan) and not with the 256x256 tiling of the same product.
+constexpr double kNarrowStepTime = 0.74, kNarrowTileTime = 2.5;
+// A split plan's second launch (splitk_reduce_kernel) beyond its traffic, in
+// steps: without it a call took 2.7 to 3.7 us less than with it where the
+// outputs are small (512 x 768, K = 3072: 22.3 / 16.3 us, 3.3 of the difference
+// traffic; 256 x 256, K = 16384: 29.9 / 26.2, 0.7 traffic).
 constexpr double kReduceLaunch = 2.0;
 
 // The kernel one NT GEMM call runs (df_fp8_gemm_nt_plan reports it): the
@@ -1293,6 +1300,7 @@ struct NtPlan {
     int split;  // K slices (1 = unsplit)
     int L;      // persistent split: DMA steps per slice
     int grid;   // persistent: blocks
+    double cost = 0.0;  // modelled time in steps (persistent and small kernels)
     SmallPlan small{0, 0, 0, 0.0};  // waves > 0: gemm_small.hip's tiles (kind PERSISTENT_NARROW, split = waves)
 };
 
@@ -1306,22 +1314,24 @@ static NtPlan nt_plan(const GemmArgs& g) {
         NtPlan wide;
         double wcost;
         if (tiles >= cus) {
-            wide = NtPlan{DF_GEMM_KERNEL_PERSISTENT, 1, 0, cus};
             wcost = (double)((tiles + cus - 1) / cus) * (nk + 3.0);
+            wide = NtPlan{DF_GEMM_KERNEL_PERSISTENT, 1, 0, cus, wcost};
         } else {
             const PSplit ps = persistent_split_plan(g.M, g.N, g.K, ws, cus);
-            wide = ps.S == 1 ? NtPlan{DF_GEMM_KERNEL_PERSISTENT, 1, 0, (int)tiles}
-                             : NtPlan{DF_GEMM_KERNEL_PERSISTENT, ps.S, ps.L, (int)std::min<int64_t>(tiles * ps.S, cus)};
             wcost = ps.cost;
+            // the reduce launch, which the choice between split and unsplit does not see
+            wide = ps.S == 1 ? NtPlan{DF_GEMM_KERNEL_PERSISTENT, 1, 0, (int)tiles, wcost}
+                             : NtPlan{DF_GEMM_KERNEL_PERSISTENT, ps.S, ps.L, (int)std::min<int64_t>(tiles * ps.S, cus),
+                                      wcost + kReduceLaunch};
         }
-        const double ncost = (double)((tiles_nw + cus - 1) / cus) * (nk * kNarrowStep + kNarrowOverhead);
-        // a split plan's second launch (the slice reduce) costs kReduceLaunch
-        // steps that the choice between split and unsplit does not see
+        const double nrounds = (double)((tiles_nw + cus - 1) / cus);
+        const double ncost = nrounds * (nk * kNarrowStep + kNarrowOverhead);
         const SmallPlan sm = small_plan(g.M, g.N, g.K, cus);
-        if (sm.cost < std::min(ncost, wcost + (wide.split > 1 ? kReduceLaunch : 0.0)) * 0.97)
-            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, sm.waves, 0, 0, sm};
+        if (sm.cost < std::min(ncost, wide.cost) * 0.97)
+            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, sm.waves, 0, 0, sm.cost, sm};
         if (ncost < wcost * 0.97)
-            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, 1, 0, (int)std::min<int64_t>(tiles_nw, cus)};
+            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, 1, 0, (int)std::min<int64_t>(tiles_nw, cus),
+                          nrounds * (nk * kNarrowStepTime + kNarrowTileTime)};
         return wide;
     }
     const GemmPlan gp = plan_gemm(g.M, g.N, g.K, ws);
@@ -1373,8 +1383,19 @@ static void launch_shape(const GemmArgs& g, int bias_dtype, int c_dtype) {
 // Grouped backward launch: dW (problem 0, in S K slices when that balances
 // better) and dX (problem 1) in one persistent grid of `cus` blocks, dealt by
 // the static schedule of gemm_sched.hpp.  The plan compares, in the rounds
-// cost model's steps, the schedule's makespan (plus the slice reduce) with
-// the two launches it replaces: dX's rounds plus dW's own plan.
+// cost model's steps, the best schedule's makespan and a fixed part with the
+// two launches it replaces, at the price of the plans that those calls run.
+// The fixed parts, unsplit and with dW in slices (the reduce launch in it),
+// are fitted: a grouped launch of few steps takes longer than its steps (344
+// tokens, 1941 -> 136, 6 steps: 24.6 us against 14.6 for the two launches;
+// 4096, 640 -> 640, seven slices, 12.6 steps: 27.1).  Over 76 sampled shapes
+// (256 to 16384 tokens, widths 64 to 6400) the choice takes 0.9% more time
+// than the better of the two forms, on average; when it priced both launches
+// at 256x256 tiles, 39% more.  us, grouped / separate: 16009 tokens, 128 -> 192
+// 36.7 / 17.0; 4096, 640 -> 640 27.1 / 19.5; 16384, 512 -> 512 38.5 / 27.8;
+// 16384, 768 -> 768 40.5 / 50.9; 16384, 1600 -> 4800 223 / 236.
+constexpr double kGroupOverhead = 1.0, kGroupSlicesOverhead = 5.0;
+
 struct GroupPlan {
     bool grouped;
     int S, L;
@@ -1388,7 +1409,6 @@ static int64_t group_makespan(int cus, int64_t units0, int c0, int64_t units1, i
 }
 
 static GroupPlan grouped_plan(const GemmArgs& dw, const GemmArgs& dx, size_t ws_bytes, int cus) {
-    constexpr double kOverheadSteps = kUnitOverhead;
     const double red_steps_per_byte = 2.0 / 10e6;
     const int nk0 = (dw.K + kPKB - 1) / kPKB, nk1 = (dx.K + kPKB - 1) / kPKB;
     // Where df_fp8_gemm_bwd_dx, given this workspace, cuts dX's reduction into
@@ -1396,23 +1416,16 @@ static GroupPlan grouped_plan(const GemmArgs& dw, const GemmArgs& dx, size_t ws_
     // waves share the reduction), dX is left to that call: the grouped launch
     // never slices dX, and this keeps dX bit-identical between the two entry
     // points.
-    GemmArgs dxs = dx;
-    dxs.ws = ws_bytes ? reinterpret_cast<float*>(uintptr_t{16}) : nullptr;  // only its presence is read
-    dxs.ws_bytes = ws_bytes;
-    if (nt_plan(dxs).split > 1) return GroupPlan{false, 1, nk0};
+    GemmArgs dxs = dx, dws = dw;
+    dxs.ws = dws.ws = ws_bytes ? reinterpret_cast<float*>(uintptr_t{16}) : nullptr;  // only its presence is read
+    dxs.ws_bytes = dws.ws_bytes = ws_bytes;
+    const NtPlan px = nt_plan(dxs);
+    if (px.split > 1) return GroupPlan{false, 1, nk0};
+    const double separate = px.cost + nt_plan(dws).cost;
     const int64_t t0 = (int64_t)((dw.M + kPBM - 1) / kPBM) * ((dw.N + kPBN - 1) / kPBN);
     const int64_t t1 = (int64_t)((dx.M + kPBM - 1) / kPBM) * ((dx.N + kPBN - 1) / kPBN);
-    // the two launches it replaces
-    double separate = (double)((t1 + cus - 1) / cus) * (nk1 + kOverheadSteps);
-    if (t0 >= cus) {
-        separate += (double)((t0 + cus - 1) / cus) * (nk0 + kOverheadSteps);
-    } else {
-        const PSplit ps = persistent_split_plan(dw.M, dw.N, dw.K, ws_bytes, cus);
-        separate += (double)((t0 * ps.S + cus - 1) / cus) * (ps.L + kOverheadSteps);
-        if (ps.S > 1) separate += (double)(ps.S + 1) * dw.M * dw.N * sizeof(float) * red_steps_per_byte;
-    }
-    GroupPlan best{false, 1, nk0};
-    double best_cost = separate;
+    GroupPlan best{true, 1, nk0};
+    double best_cost = 1e300;
     for (int s = 1; s <= 8; ++s) {
         const int span = (nk0 + s - 1) / s;
         if (s > 1 && span < 4) break;
@@ -1425,7 +1438,8 @@ static GroupPlan grouped_plan(const GemmArgs& dw, const GemmArgs& dx, size_t ws_
             best = GroupPlan{true, se, span};
         }
     }
-    return best;
+    best_cost += best.S > 1 ? kGroupSlicesOverhead : kGroupOverhead;
+    return best_cost < separate ? best : GroupPlan{false, 1, nk0};
 }
 
 // amax_part non-NULL: the launch also folds |dX| into 8 partials per block

@@ -322,6 +322,19 @@ def test_grouped_backward_shapes(dev, M, K, N):
     grouped_case(dev, M, K, N, seed=M + 3 * K + 7 * N, out16=True)
 
 
+# M, K, N and whether the grouped launch is the faster form (both measured;
+# the times stand beside the rule in csrc/gemm_fp8.hip)
+@pytest.mark.parametrize("M,K,N,grouped", [(16009, 128, 192, False), (16384, 256, 256, False), (4096, 640, 640, False),
+                                           (344, 1941, 136, False), (16384, 768, 768, True), (5000, 1037, 771, True),
+                                           (16384, 1600, 4800, True)])
+def test_backward_takes_the_faster_form(dev, M, K, N, grouped):
+    """The grouped launch is priced against the two launches that the
+    separate calls run (narrow and small tiles among them); either form
+    gives the same dX and the oracle's dW."""
+    assert df.gemm_bwd_plan(M, N, K)[0] == grouped
+    grouped_case(dev, M, K, N, seed=M + 5 * K + 11 * N, rows="bands", wrows="bands", wcols="bands")
+
+
 def test_grouped_backward_without_workspace(dev):
     """No workspace: dW cannot be sliced, the plan falls back or groups
     unsplit, and the outputs still match."""
