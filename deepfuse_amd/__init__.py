@@ -386,10 +386,13 @@ class GemmKernel(enum.IntEnum):
     TILED_REG_256 = 3
     TILED_REG_128 = 4
     PERSISTENT_NARROW = 5
+    SMALL_16 = 6
+    SMALL_32 = 7
 
 
 def gemm_plan(M: int, N: int, K: int, lda: int, ldb: int, bias=None, ws_bytes: int = 0):
-    """(GemmKernel, K slices) that df_fp8_gemm_nt takes for these arguments;
+    """(GemmKernel, K slices) that df_fp8_gemm_nt takes for these arguments
+    (SMALL_*: the waves of a block, which share the K steps);
     ``bias`` is the bias tensor the call would pass (its alignment counts)."""
     k, s = _c_int(), _c_int()
     call("df_fp8_gemm_nt_plan", M, N, K, lda, ldb, _ptr(bias), ws_bytes, ctypes.byref(k), ctypes.byref(s))

@@ -1290,9 +1290,9 @@ constexpr double kReduceLaunch = 2.0;
 // The kernel one NT GEMM call runs (df_fp8_gemm_nt_plan reports it): the
 // persistent kernel when its offsets fit (split into K-slice units when the
 // output has fewer tiles than CUs and a workspace allows it; its 256x128
-// tiles, or the small tiles of gemm_small.hip, when the rounds cost model
-// puts them 3% below), otherwise the
-// tiled kernels -- LDS-DMA when both operands fit a 32-bit buffer range,
+// tiles when the rounds cost model puts them 3% below), or the small-tile
+// kernel of gemm_small.hip when the model puts that 3% below both, otherwise
+// the tiled kernels -- LDS-DMA when both operands fit a 32-bit buffer range,
 // register-staged beyond -- with 256x256 or 128x128 blocks and split-K from
 // plan_gemm.  Every launch below follows this plan.
 struct NtPlan {
@@ -1301,7 +1301,7 @@ struct NtPlan {
     int L;      // persistent split: DMA steps per slice
     int grid;   // persistent: blocks
     double cost = 0.0;  // modelled time in steps (persistent and small kernels)
-    SmallPlan small{0, 0, 0, 0.0};  // waves > 0: gemm_small.hip's tiles (kind PERSISTENT_NARROW, split = waves)
+    SmallPlan small{0, 0, 0, 0.0};  // of the small kinds (split = its waves)
 };
 
 static NtPlan nt_plan(const GemmArgs& g) {
@@ -1328,7 +1328,7 @@ static NtPlan nt_plan(const GemmArgs& g) {
         const double ncost = nrounds * (nk * kNarrowStep + kNarrowOverhead);
         const SmallPlan sm = small_plan(g.M, g.N, g.K, cus);
         if (sm.cost < std::min(ncost, wide.cost) * 0.97)
-            return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, sm.waves, 0, 0, sm.cost, sm};
+            return NtPlan{sm.mt == 1 ? DF_GEMM_KERNEL_SMALL_16 : DF_GEMM_KERNEL_SMALL_32, sm.waves, 0, 0, sm.cost, sm};
         if (ncost < wcost * 0.97)
             return NtPlan{DF_GEMM_KERNEL_PERSISTENT_NARROW, 1, 0, (int)std::min<int64_t>(tiles_nw, cus),
                           nrounds * (nk * kNarrowStepTime + kNarrowTileTime)};
@@ -1350,7 +1350,7 @@ static NtPlan nt_plan(const GemmArgs& g) {
 template <int FA, int FB, typename OutT, typename BiasT>
 static void launch_shape(const GemmArgs& g, int bias_dtype, int c_dtype) {
     const NtPlan p = nt_plan(g);
-    if (p.small.waves) {
+    if (p.kind == DF_GEMM_KERNEL_SMALL_16 || p.kind == DF_GEMM_KERNEL_SMALL_32) {
         launch_small(p.small, FA, FB, bias_dtype, c_dtype, g);
         return;
     }

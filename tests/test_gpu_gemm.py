@@ -219,7 +219,7 @@ def test_config3_forward_bf16(dev, K, N):
 # (M, N, K) whose plan takes the persistent kernel's 256x128 tiles, with
 # ragged edges: rows and columns ending inside a wave's 64x64 part, an
 # odd-length bf16 bias, outputs whose row pitch is not 16-byte aligned.
-NARROW_CASES = [(1000, 999, 640), (1000, 1000, 768), (300, 130, 1024), (2048, 640, 2048)]
+NARROW_CASES = [(1000, 999, 640), (1000, 1000, 768), (2500, 1537, 768), (5000, 386, 1024)]
 
 
 @pytest.mark.parametrize("M,N,K", NARROW_CASES)
@@ -235,8 +235,8 @@ def test_narrow_tiles_match_oracle(dev, M, N, K):
     bq, _, sb, Bd = quant_operand(B, Fmt.E4M3, dev)
     bd = torch.from_numpy(bb.view(np.int16)).to(dev).view(torch.bfloat16)
     for ws_bytes in (0, int(df.lib().df_fp8_gemm_workspace_bytes(M, N, K))):
-        kind = df.gemm_plan(M, N, K, aq.stride(0), bq.stride(0), bd, ws_bytes)[0]
-        assert kind == df.GemmKernel.PERSISTENT_NARROW, f"plan {kind!r} (workspace {ws_bytes})"
+        plan = df.gemm_plan(M, N, K, aq.stride(0), bq.stride(0), bd, ws_bytes)
+        assert plan == (df.GemmKernel.PERSISTENT_NARROW, 1), f"plan {plan!r} (workspace {ws_bytes})"
     Y = df.gemm_nt(aq, Fmt.E4M3, bq, Fmt.E4M3, K, sa, sb, bias=bd)
     Y16 = df.gemm_nt(aq, Fmt.E4M3, bq, Fmt.E4M3, K, sa, sb, bias=bd, out_dtype=torch.bfloat16)
     check_bf16_image(Y, Y16)
@@ -255,15 +255,24 @@ def test_config4_forward_backward(dev, K, N):
     forward_case(dev, M, K, N, seed=synth.SEED_BASE + 40 + K + N, rows="bands")
 
 
-@pytest.mark.parametrize("M,N,K", [(1600, 1600, 16384), (384, 200, 8192), (4800, 1600, 16384)])
-def test_split_k_matches_unsplit(dev, M, N, K):
+@pytest.mark.parametrize("M,N,K,slices", [(1600, 1600, 16384, 5), (384, 200, 8192, 0), (4800, 1600, 16384, 0),
+                                          (1025, 1030, 8000, 7), (2049, 770, 8200, 6)])
+def test_split_k_matches_unsplit(dev, M, N, K, slices):
     """Long reductions on small outputs take the split-K path when a
-    workspace is given; without one the same product runs unsplit.  Both
-    must meet the bar against the oracle (sampled rows) and agree closely."""
+    workspace is given (`slices` K slices); without one the same product runs
+    on another plan.  Both must meet the bar against the oracle (sampled
+    rows) and agree closely.  slices 0: outputs so small that the small tiles
+    take them, or too large to split, workspace or not."""
     A = synth.normal((M, K), 1e-3, seed=M + N)
     B = synth.normal((N, K), 1.0, seed=M + N + 1)
     aq, _, sa, Ad = quant_operand(A, Fmt.E5M2, dev)
     bq, _, sb, Bd = quant_operand(B, Fmt.E4M3, dev)
+    plans = [df.gemm_plan(M, N, K, aq.stride(0), bq.stride(0), None, b) for b in (1 << 30, 0)]
+    if slices:
+        assert plans[0] == (df.GemmKernel.PERSISTENT, slices) and plans[1][0] != df.GemmKernel.PERSISTENT, plans
+        assert df.lib().df_fp8_gemm_workspace_bytes(M, N, K) >= 4 * slices * M * N
+    else:
+        assert plans[0] == plans[1], plans
     with_ws = df.gemm_nt(aq, Fmt.E5M2, bq, Fmt.E4M3, K, sa, sb).cpu().numpy()
     no_ws = df.gemm_nt(aq, Fmt.E5M2, bq, Fmt.E4M3, K, sa, sb, split_k=False).cpu().numpy()
     idx = np.sort(np.random.default_rng(M).choice(M, 16, replace=False))
@@ -271,8 +280,6 @@ def test_split_k_matches_unsplit(dev, M, N, K):
     assert orc.rel_err(with_ws[idx], ref) <= TOL
     assert orc.rel_err(no_ws[idx], ref) <= TOL
     assert orc.rel_err(with_ws, no_ws) <= 1e-5
-    if (M, N) in ((1600, 1600), (384, 200)):
-        assert df.lib().df_fp8_gemm_workspace_bytes(M, N, K) > 0  # these two do take split-K
 
 
 def grouped_case(dev, M, K, N, seed, rows=None, wrows=None, wcols=None, out16=False):

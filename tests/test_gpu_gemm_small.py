@@ -20,15 +20,16 @@ from test_gpu_gemm import TOL, band_rows, check_bf16_image, quant_operand
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K, and whether the tiling is 16x16 (else 32x32)
-CASES = [(1, 1, 5), (1, 17, 128), (15, 16, 144), (16, 33, 127), (17, 1601, 272), (8, 1600, 1600), (8, 640, 6400),
-         (31, 2049, 640), (32, 2048, 512), (33, 3072, 784), (64, 3072, 768), (63, 1600, 3072), (97, 130, 2064),
-         (512, 768, 768), (300, 257, 1040)]
+# M, N, K, the tile and the waves of a block
+CASES = [(1, 1, 5, 16, 4), (1, 17, 128, 16, 4), (15, 16, 144, 16, 4), (16, 33, 127, 16, 4), (17, 1601, 272, 32, 4),
+         (8, 1600, 1600, 16, 4), (8, 640, 6400, 16, 4), (31, 2049, 640, 32, 4), (32, 2048, 512, 32, 4),
+         (33, 3072, 784, 32, 4), (64, 3072, 768, 32, 4), (63, 1600, 3072, 16, 4), (97, 130, 2064, 16, 4),
+         (512, 768, 768, 32, 4), (300, 257, 1040, 32, 8), (300, 130, 1024, 16, 4), (2048, 640, 2048, 32, 4)]
 
 
-@pytest.mark.parametrize("M,N,K", CASES)
+@pytest.mark.parametrize("M,N,K,tile,waves", CASES)
 @pytest.mark.parametrize("fa,fb", [(Fmt.E4M3, Fmt.E4M3), (Fmt.E5M2, Fmt.E4M3)])
-def test_small_tiles_match_oracle(dev, M, N, K, fa, fb):
+def test_small_tiles_match_oracle(dev, M, N, K, tile, waves, fa, fb):
     seed = synth.SEED_BASE + 31 * M + 7 * N + K
     A = synth.normal((M, K), 1.0, seed=seed)
     B = synth.normal((N, K), 0.02, seed=seed + 1)
@@ -42,8 +43,8 @@ def test_small_tiles_match_oracle(dev, M, N, K, fa, fb):
         dst[:, :kp].copy_(src)
     aq, bq = wide[0][:, :kp], wide[1][:, :kp]
     bd = torch.from_numpy(bb.view(np.int16)).to(dev).view(torch.bfloat16)
-    kind, split = df.gemm_plan(M, N, K, aq.stride(0), bq.stride(0), bd, 1 << 30)
-    assert kind == df.GemmKernel.PERSISTENT_NARROW and split > 1, f"plan {kind!r} {split}"
+    plan = df.gemm_plan(M, N, K, aq.stride(0), bq.stride(0), bd, 1 << 30)
+    assert plan == (df.GemmKernel.SMALL_16 if tile == 16 else df.GemmKernel.SMALL_32, waves), f"plan {plan!r}"
     Y = df.gemm_nt(aq, fa, bq, fb, K, sa, sb, bias=bd)
     ref = orc.fc_forward(Ad, Bd, orc.bf16_to_f32(bb))
     err = orc.rel_err(Y.cpu().numpy(), ref)
