@@ -5,8 +5,9 @@ path's bar (1e-4), on every row.
 
 Shapes: one value short of, on and past the tile edges (16, 32) in M and N;
 K within one step, on a step's edge, one 16-byte chunk past it, not a
-multiple of 16, fewer steps than waves and more than one round of them;
-outputs whose rows are not 16-byte aligned; both widths of the wave count.
+multiple of 16, fewer steps than waves; more than one round of steps (a wave's
+slab written again after it was read) for each tiling and wave count, whole
+rounds and a partial last one; outputs whose rows are not 16-byte aligned.
 The operands' leading dimensions hold codes past K that must not be read.
 """
 import numpy as np
@@ -24,7 +25,8 @@ pytestmark = pytest.mark.gpu
 CASES = [(1, 1, 5, 16, 4), (1, 17, 128, 16, 4), (15, 16, 144, 16, 4), (16, 33, 127, 16, 4), (17, 1601, 272, 32, 4),
          (8, 1600, 1600, 16, 4), (8, 640, 6400, 16, 4), (31, 2049, 640, 32, 4), (32, 2048, 512, 32, 4),
          (33, 3072, 784, 32, 4), (64, 3072, 768, 32, 4), (63, 1600, 3072, 16, 4), (97, 130, 2064, 16, 4),
-         (512, 768, 768, 32, 4), (300, 257, 1040, 32, 8), (300, 130, 1024, 16, 4), (2048, 640, 2048, 32, 4)]
+         (512, 768, 768, 32, 4), (300, 257, 1040, 32, 8), (300, 130, 1024, 16, 4), (2048, 640, 2048, 32, 4),
+         (512, 768, 3072, 32, 4), (1000, 771, 1037, 32, 4), (512, 512, 3088, 32, 8), (255, 769, 3072, 32, 8)]
 
 
 @pytest.mark.parametrize("M,N,K,tile,waves", CASES)
