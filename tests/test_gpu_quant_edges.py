@@ -80,8 +80,8 @@ def test_edges(dev, rows, cols, dt, fmt):
 @pytest.mark.parametrize("affine", [True, False])
 def test_layernorm_codes(dev, rows, cols, dt, affine):
     """The fused LayerNorm's codes and scale are those of the quantize of its
-    own y, and y is within rounding of binary64 (a NaN row, a constant row and
-    values that overflow the element type among them)."""
+    own y, and y is within rounding of binary64 (a NaN row and a constant row
+    among them)."""
     g = torch.Generator().manual_seed(rows + 31 * cols)
     x = torch.randn(rows, cols, generator=g) * 2 + 0.25
     if rows > 4:
@@ -107,6 +107,33 @@ def test_layernorm_codes(dev, rows, cols, dt, affine):
     err = (y.double() - ref).abs()[ok]
     bound = ulp * ref.abs()[ok] + cols * 2.0 ** -24 * 8 + 2.0 ** -25
     assert bool((err <= bound).all()) and bool(torch.isnan(y[~ok]).all())
+
+
+@pytest.mark.parametrize("rows,cols", [(130, 1600), (33, 771), (9, 2056), (20, 3001)])
+@pytest.mark.parametrize("dt", [F32, BF16, F16])
+def test_layernorm_codes_overflow(dev, rows, cols, dt):
+    """Values that overflow the element type when y is rounded to it: infinite
+    in y, left out of the absmax, saturated as codes.  Columns with a gamma
+    that takes most values past the range, and columns whose beta is the
+    largest finite value and whose gamma is about its unit in the last place:
+    y is rounded to that value on one side of it, to infinity on the other."""
+    g = torch.Generator().manual_seed(rows + 7 * cols)
+    x = (torch.randn(rows, cols, generator=g) * 2 + 0.25).to(dt).to(dev)
+    gamma, beta = torch.ones(cols), torch.zeros(cols)
+    top = torch.finfo(dt).max
+    gamma[::97] = top / 1.5
+    gamma[5::97], beta[5::97] = {F32: 2.0e31, BF16: 1.4e36, F16: 32.0}[dt], top
+    gamma, beta = gamma.to(dt).to(dev), beta.to(dt).to(dev)
+    y0 = df.layernorm(x, gamma, beta)
+    h = host(y0)
+    assert np.isinf(h[:, ::97]).any() and np.isinf(h[:, 5::97]).any() and (h[:, 5::97] == top).any()
+    s = orc.scale(orc.absmax(h), int(Fmt.E4M3))
+    y, q, qt, sc = df.layernorm(x, gamma, beta, fmt=Fmt.E4M3, want_y=True, want_qt=True)
+    bits = torch.int32 if dt == F32 else torch.int16
+    assert torch.equal(y.view(bits), y0.view(bits)) and sc.item() == np.float32(s)
+    codes = orc.quantize(h, s, int(Fmt.E4M3))
+    assert np.array_equal(q.cpu().numpy()[:, :cols], codes)
+    assert np.array_equal(qt.cpu().numpy()[:, :rows], codes.T)
 
 
 # one and three partials past the count (8192) up to which every tile block of
