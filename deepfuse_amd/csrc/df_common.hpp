@@ -49,21 +49,13 @@ __device__ __forceinline__ uint32_t fold_f32(uint32_t m, uint32_t bits) {
     return max(m, a < 0x7F800000u ? a : 0u);
 }
 
-// two bf16 in one dword: widen each to its binary32 pattern
-__device__ __forceinline__ uint32_t fold_bf16x2(uint32_t m, uint32_t w) {
-    const uint32_t hi = w & 0x7FFF0000u;
-    const uint32_t lo = (w << 16) & 0x7FFF0000u;
-    m = max(m, hi < 0x7F800000u ? hi : 0u);
-    return max(m, lo < 0x7F800000u ? lo : 0u);
-}
-
-// The same folds without compares, for code whose VALU slots are scarce (a
+// The same fold without compares, for code whose VALU slots are scarce (a
 // compare's lane mask read by the next VALU instruction costs wait states).
 // Adding 0x00800000 to a sign-cleared binary32 pattern (0x0080 to each
 // sign-cleared bf16 half of a dword: no carry crosses the halves) maps finite
 // patterns to positive and inf/NaN patterns to negative signed values, so a
 // signed max that starts at 0 skips the latter.  unbias_* turns such an
-// accumulator back into the binary32 pattern fold_f32 / fold_bf16x2 give.
+// accumulator back into the binary32 pattern that fold_f32 gives.
 __device__ __forceinline__ uint32_t fold_f32_biased(uint32_t m, uint32_t bits) {
     return (uint32_t)max((int)m, (int)((bits & 0x7FFFFFFFu) + 0x00800000u));
 }

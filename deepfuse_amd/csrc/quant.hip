@@ -49,7 +49,7 @@ template <bool NT, typename T> __device__ __forceinline__ void st_nt(T* p, const
 }
 
 // ------------------------------------------------------------------ absmax --
-// (fold_f32 and fold_bf16x2, the binary32 and bf16-pair folds, are in df_common.hpp)
+// (the folds of |x| are in df_common.hpp)
 
 __device__ __forceinline__ uint32_t block_max_u32(uint32_t m) {
     __shared__ uint32_t red[kThreads / 64];
