@@ -482,6 +482,7 @@ def measured_traffic(kernel_family):
         return None, None
 
 
+SMALL_CALLS = ("linear_fp32_64", "decode_xl_8", "step_small_512", "step_ragged_f16")
 # The profiling runs behind profiles/ (from the repository root on one
 # MI355X, with TMPDIR=/tmp), and the directories they write.
 PROFILE_COMMANDS = {
@@ -531,6 +532,10 @@ PROFILE_COMMANDS = {
     "stats_producer": ("rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/prof_producer -o bench "
                        "-- python3 bench.py --steps 2 --warmup 1 --no-cpu-baseline --no-conversion --no-streaming "
                        "--no-optimizer --no-delayed --no-config3"),
+    "stats_small": ("rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/prof_small -o bench -- "
+                    "python3 -c \"import torch; from perf import cases as c; "
+                    "[(s := c.prepare(k, 1), [c.run(s) for _ in range(20)], torch.cuda.synchronize()) "
+                    "for k in c.listed() if k['name'] in '" + " ".join(SMALL_CALLS) + "'.split()]\""),
     "stats_config3": ("rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/prof_config3 -o bench "
                       "-- python3 bench.py --config3-only"),
 }
@@ -542,11 +547,18 @@ EXTRA_STATS = (
      ("adam_kernel", "sumsq_kernel", "clip_kernel", "norm_finalize_kernel")),
     ("stats_producer", "prof_producer", "layernorm_quantize_kernel_stats.md",
      "LayerNorm + e4m3 codes, 16384 x 1600 bf16 (unfused chain, fused, fused delayed)",
-     ("ln_stats_", "true>(unsigned short const*", "true, false>(unsigned short const*", "amax_history_kernel")),
+     ("ln_stats_", "quantize_2d_kernel<unsigned short, 0, false, true, false, true, true>",
+      "quantize_2d_kernel<unsigned short, 0, false, true, true, true, false>",
+      "quantize_2d_kernel<unsigned short, 0, false, false, false, true, false>", "amax_history_kernel")),
     ("stats_producer", "prof_producer", "gemm_producer_kernel_stats.md",
      "GEMMs that also fold their output's absmax: fc1's forward and fc2's grouped backward at the config-4 fc "
      "shapes (the producer leg's gemm_producer variants)",
      ("persistent_amax_kernel", "grouped_amax_kernel")),
+    ("stats_small", "prof_small", "small_calls_kernel_stats.md",
+     "small and ragged calls of perf/cases.py (" + ", ".join(SMALL_CALLS) + "), 20 passes each",
+     ("gemm_small_kernel", "quantize_2d_small_kernel", "quantize_2d_jit_w5_kernel", "absmax_colsum_stage1",
+      "absmax_f16_stage1", "absmax_f32_stage1", "absmax_bf16_stage1", "narrow_kernel", "gemm_nt_persistent_kernel",
+      "colsum_reduce_kernel", "batch")),
 )
 # GEMM families whose C-ABI call is exactly one kernel, by the persistent
 # kernel's template arguments: <A format, B format, output, bias type, bias,
@@ -770,7 +782,7 @@ def summarize_profiles():
             rows_x = [r for r in csv.DictReader(fh) if any(k in r["Name"] for k in keep)]
         lines = [f"# rocprofv3 kernel statistics -- {title}", "",
                  "Command (from the repository root, on one MI355X):", "", "    " + PROFILE_COMMANDS[key], "",
-                 "Only this leg's own kernels are listed (the config-4 step also runs in the same process).  "
+                 "Only this leg's own kernels are listed (others run in the same process).  "
                  "Durations in microseconds.", "",
                  "| kernel | calls | avg us | min us | max us |", "|---|---|---|---|---|"]
         for r in rows_x:

@@ -15,10 +15,10 @@
 // LDS and are added in wave order, so the result does not depend on timing.
 // No second launch adds K slices up.  Measured, against the persistent
 // kernel's tiles (us a call; bf16 output):
-//       8 x 1600, K = 1600    3.9  against 16.8    8 x 6400, K = 1600   5.3  against 17.5
-//       8 x 1600, K = 6400    6.6  against 21.0   64 x 3072, K = 768    4.0  against  8.1
-//     512 x 768,  K = 768     4.9  against  8.5  512 x 768,  K = 3072   8.3  against 23.1
-//    1000 x 771,  K = 1037    9.0  against 15.6  768 x 768,  K = 8192  21.2  against 30.6
+//       8 x 1600, K = 1600    3.3  against 16.4    8 x 6400, K = 1600   4.8  against 17.3
+//       8 x 1600, K = 6400    6.1  against 20.6   64 x 3072, K = 768    3.5  against  7.3
+//     512 x 768,  K = 768     4.3  against  7.7  512 x 768,  K = 3072   7.5  against 22.6
+//    1000 x 771,  K = 1037    8.6  against 14.5  768 x 768,  K = 8192  20.6  against 30.8
 //
 // Operand path: each load instruction takes 8 rows x 128 bytes, whole cache
 // lines, into registers; a wave-private LDS slab turns them into MFMA
@@ -194,9 +194,12 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(
 // tiles were measured too and were nowhere faster by more than 5%: their
 // blocks are too few where the latency counts, and where bytes count the
 // persistent kernel is ahead.  32x32 tiles run eight waves instead of four
-// where that shortens the chain and the blocks do not fill the CUs anyway
-// (64 x 1600, K = 6400: 9.0 against 10.6 us; 512 x 768, K = 768, 384 blocks:
-// 5.8 against 4.9).
+// where the blocks do not fill the CUs anyway and a wave of four would have
+// more than one round of steps.  Eight / four waves, us: 128 x 1600, K = 6400
+// (200 blocks, 50 steps) 10.3 / 11.1; 96 x 1600, K = 6400 8.7 / 9.7; 128 x 1600,
+// K = 1600 (13 steps) 5.40 / 5.46; near a full chip at 24 steps four are a
+// little ahead (512 x 512, K = 3072, 256 blocks: 5.43 / 5.26), and past it
+// clearly (512 x 768, K = 3072, 384 blocks: 8.6 / 7.2).
 SmallPlan small_plan(int M, int N, int K, int cus) {
     const double nk = (K + 127) / 128;
     const double b16 = (double)((M + 15) / 16) * ((N + 15) / 16), b32 = (double)((M + 31) / 32) * ((N + 31) / 32);
