@@ -482,6 +482,13 @@ def measured_traffic(kernel_family):
         return None, None
 
 
+def _cases_cmd(names, passes):
+    """A python command that runs cases of perf/cases.py."""
+    return ("python3 -c \"import torch; from perf import cases as c; "
+            f"[(s := c.prepare(k, 1), [c.run(s) for _ in range({passes})], torch.cuda.synchronize()) "
+            f"for k in c.listed() if k['name'] in '{' '.join(names)}'.split()]\"")
+
+
 SMALL_CALLS = ("linear_fp32_64", "decode_xl_8", "step_small_512", "step_ragged_f16")
 # The profiling runs behind profiles/ (from the repository root on one
 # MI355X, with TMPDIR=/tmp), and the directories they write.
@@ -533,9 +540,11 @@ PROFILE_COMMANDS = {
                        "-- python3 bench.py --steps 2 --warmup 1 --no-cpu-baseline --no-conversion --no-streaming "
                        "--no-optimizer --no-delayed --no-config3"),
     "stats_small": ("rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/prof_small -o bench -- "
-                    "python3 -c \"import torch; from perf import cases as c; "
-                    "[(s := c.prepare(k, 1), [c.run(s) for _ in range(20)], torch.cuda.synchronize()) "
-                    "for k in c.listed() if k['name'] in '" + " ".join(SMALL_CALLS) + "'.split()]\""),
+                    + _cases_cmd(SMALL_CALLS, 20)),
+    "pmc_cases": ("timeout -s KILL 180 rocprofv3 --pmc SQ_WAVES SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_WAIT_INST_ANY "
+                  "SQ_ACTIVE_INST_VALU SQ_INSTS_VALU GRBM_GUI_ACTIVE --kernel-trace "
+                  "--output-format csv -d gpurun_out/pmc_cases -o bench -- "
+                  + _cases_cmd(("layernorm_xl",) + SMALL_CALLS, 2)),
     "stats_config3": ("rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/prof_config3 -o bench "
                       "-- python3 bench.py --config3-only"),
 }
@@ -797,6 +806,8 @@ def summarize_profiles():
         extra.append("gemm_tile_timeline_config4.md")
     if limiter_summary(out_dir, prof):
         extra.append("limiters_config4.md")
+    if case_counter_summary(out_dir, prof):
+        extra.append("limiters_small_and_layernorm.md")
     if config3_summary(out_dir, prof):
         extra.append("gemm_config3_kernels.md")
     print(f"wrote profiles/ summaries ({len(rows)} kernels, traffic families {sorted(fams)}, extra {extra})")
@@ -1151,6 +1162,53 @@ def limiter_summary(out_dir, prof):
     row("fabric read requests per dispatch", lambda a: a["TCC_EA0_RDREQ_sum"], "{:.0f}")
     row("fabric write requests per dispatch", lambda a: a["TCC_EA0_WRREQ_sum"], "{:.0f}")
     with open(os.path.join(prof, "limiters_config4.md"), "w") as fh:
+        fh.write("\n".join(lines) + "\n")
+    return True
+
+
+CASE_KERNELS = (  # the row's label and the start of the kernel's name
+    ("LayerNorm statistics, whole chunks, bf16", "void dfk::ln_stats_whole_kernel<unsigned short, true>"),
+    ("LayerNorm tiles to codes, bf16", "void dfk::quantize_2d_kernel<unsigned short, 0, false, true, false, true, true>"),
+    ("GEMM on 16x16 tiles", "void dfk::gemm_small_kernel<0, 0, 1, 1, 4, 4>"),
+    ("GEMM on 32x32 tiles", "void dfk::gemm_small_kernel<0, 0, 2, 2, 4, 2>"),
+    ("quantize, one launch, bf16", "void dfk::quantize_2d_small_kernel<unsigned short, 0, true>"),
+    ("quantize, few tiles, bf16", "void dfk::quantize_2d_small_kernel<unsigned short, 0, false>"),
+    ("absmax with column sums, bf16 (512 rows)", "void dfk::absmax_colsum_stage1<unsigned short>"),
+)
+
+
+def case_counter_summary(out_dir, prof):
+    """profiles/limiters_small_and_layernorm.md from the pmc_cases run:
+    averages per dispatch; SQ_WAVE_CYCLES and SQ_ACTIVE_INST_VALU count
+    quad-cycles, GRBM_GUI_ACTIVE once per XCD."""
+    import csv
+
+    path = os.path.join(out_dir, "pmc_cases", "bench_counter_collection.csv")
+    if not os.path.exists(path):
+        return False
+    vals = {}
+    with open(path) as fh:
+        for r in csv.DictReader(fh):
+            for label, pre in CASE_KERNELS:
+                if r["Kernel_Name"].startswith(pre):
+                    vals.setdefault(label, {}).setdefault(r["Counter_Name"], []).append(float(r["Counter_Value"]))
+    lines = ["# What bounds LayerNorm to codes and the kernels of small calls -- rocprofv3 counters", "",
+             "Command (from the repository root, on one MI355X):", "", "    " + PROFILE_COMMANDS["pmc_cases"], "",
+             "Averages per dispatch, the kernels one at a time.  VALU cycles = 4 x SQ_ACTIVE_INST_VALU over 1024 SIMDs; "
+             "waiting and ready but not issued as fractions of SQ_WAVE_CYCLES; a wave's cycles = 4 x SQ_WAVE_CYCLES over "
+             "SQ_WAVES.  window = GRBM_GUI_ACTIVE / 8: under counter collection it is some 20000 cycles longer than "
+             "these short kernels, whose times stand in the kernel statistics.", "",
+             "| kernel | waves | a wave's cycles | VALU instructions per wave | VALU cycles per SIMD | window | waiting "
+             "(s_waitcnt, barrier) | ready, not issued |", "|---|---|---|---|---|---|---|---|"]
+    for label, pre in CASE_KERNELS:
+        if label not in vals:
+            continue
+        a = {c: sum(v) / len(v) for c, v in vals[label].items()}
+        cyc, wc = a["GRBM_GUI_ACTIVE"] / 8, a["SQ_WAVE_CYCLES"]
+        lines.append(f"| {label} (`{pre[len('void dfk::'):]}`) | {a['SQ_WAVES']:.0f} | {4 * wc / a['SQ_WAVES']:.0f} | "
+                     f"{a['SQ_INSTS_VALU'] / a['SQ_WAVES']:.0f} | {4 * a['SQ_ACTIVE_INST_VALU'] / 1024:.0f} | "
+                     f"{cyc:.0f} | {a['SQ_WAIT_ANY'] / wc:.3f} | {a['SQ_WAIT_INST_ANY'] / wc:.3f} |")
+    with open(os.path.join(prof, "limiters_small_and_layernorm.md"), "w") as fh:
         fh.write("\n".join(lines) + "\n")
     return True
 
