@@ -190,7 +190,10 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(
 // fixed part (partial tiles, output) plus the K steps' operand bytes:
 //   16x16 tiles, 4 waves: 2.5 + 0.06 nk + (blocks / CUs) * (0.75 + 0.031 nk) us
 //   32x32 tiles:          2.6 + 0.11 nk + (blocks / CUs) * (0.75 + 0.080 nk) us
-// within 10-15% from 8 to 2048 rows, K = 512 to 6400.  16x32, 32x64 and 64x64
+// within 10-15% from 8 to 2048 rows, K = 512 to 6400.  Longer reductions stream
+// operand panels that no L2 holds, and 16x16 tiles, which take in twice the bytes
+// of 32x32 ones, then cost more a step: 0.045 nk (102 x 1808, K = 12112: 31.8 us on
+// 16x16 tiles, 19.6 on 32x32, 28.3 on the persistent kernel's).  16x32, 32x64 and 64x64
 // tiles were measured too and were nowhere faster by more than 5%: their
 // blocks are too few where the latency counts, and where bytes count the
 // persistent kernel is ahead.  32x32 tiles run eight waves instead of four
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(64 * W) void gemm_small_kernel(
 SmallPlan small_plan(int M, int N, int K, int cus) {
     const double nk = (K + 127) / 128;
     const double b16 = (double)((M + 15) / 16) * ((N + 15) / 16), b32 = (double)((M + 31) / 32) * ((N + 31) / 32);
-    const double t16 = 2.5 + 0.06 * nk + b16 / cus * (0.75 + 0.031 * nk);
+    const double t16 = 2.5 + 0.06 * nk + b16 / cus * (0.75 + (nk > 50 ? 0.045 : 0.031) * nk);
     const double t32 = 2.6 + 0.11 * nk + b32 / cus * (0.75 + 0.080 * nk);
     if (t16 < t32) return SmallPlan{1, 1, 4, t16 / kStepUs};
     return SmallPlan{2, 2, b32 <= cus && nk > 8 ? 8 : 4, t32 / kStepUs};

@@ -26,7 +26,8 @@ CASES = [(1, 1, 5, 16, 4), (1, 17, 128, 16, 4), (15, 16, 144, 16, 4), (16, 33, 1
          (8, 1600, 1600, 16, 4), (8, 640, 6400, 16, 4), (31, 2049, 640, 32, 4), (32, 2048, 512, 32, 4),
          (33, 3072, 784, 32, 4), (64, 3072, 768, 32, 4), (63, 1600, 3072, 16, 4), (97, 130, 2064, 16, 4),
          (512, 768, 768, 32, 4), (300, 257, 1040, 32, 8), (300, 130, 1024, 16, 4), (2048, 640, 2048, 32, 4),
-         (512, 768, 3072, 32, 4), (1000, 771, 1037, 32, 4), (512, 512, 3088, 32, 8), (255, 769, 3072, 32, 8)]
+         (512, 768, 3072, 32, 4), (1000, 771, 1037, 32, 4), (512, 512, 3088, 32, 8), (255, 769, 3072, 32, 8),
+         (102, 1808, 12112, 32, 8), (102, 200, 12112, 16, 4)]
 
 
 @pytest.mark.parametrize("M,N,K,tile,waves", CASES)
