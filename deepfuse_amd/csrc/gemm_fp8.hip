@@ -1388,13 +1388,19 @@ static void launch_shape(const GemmArgs& g, int bias_dtype, int c_dtype) {
 // The fixed parts, unsplit and with dW in slices (the reduce launch in it),
 // are fitted: a grouped launch of few steps takes longer than its steps (344
 // tokens, 1941 -> 136, 6 steps: 24.6 us against 14.6 for the two launches;
-// 4096, 640 -> 640, seven slices, 12.6 steps: 27.1).  Over 76 sampled shapes
-// (256 to 16384 tokens, widths 64 to 6400) the choice takes 0.9% more time
-// than the better of the two forms, on average; when it priced both launches
-// at 256x256 tiles, 39% more.  us, grouped / separate: 16009 tokens, 128 -> 192
-// 36.7 / 17.0; 4096, 640 -> 640 27.1 / 19.5; 16384, 512 -> 512 38.5 / 27.8;
-// 16384, 768 -> 768 40.5 / 50.9; 16384, 1600 -> 4800 223 / 236.
-constexpr double kGroupOverhead = 1.0, kGroupSlicesOverhead = 5.0;
+// 4096, 640 -> 640, seven slices, 12.6 steps: 27.1).  A dX of few K steps is
+// bound by its stores, which a grouped launch puts beside dW's steps and a
+// separate one does not: at least its bytes (two an element) at 2.5 TB/s, 1
+// TB/s where its rows leave 16-byte stores no room (12112 x 1808, K = 102 19.7
+// us for 44 MB, 16384 x 1600, K = 64 16.4 for 52; 15313 x 1322, K = 64 55 for
+// 40).  Over 76 sampled shapes (256 to 16384 tokens, widths 64 to 6400) the
+// choice takes 0.9% more time than the better of the two forms, on average;
+// when it priced both launches at 256x256 tiles, 39% more.  us, grouped /
+// separate: 16009 tokens, 128 -> 192 36.7 / 17.0; 4096, 640 -> 640 27.1 / 19.5;
+// 16384, 512 -> 512 38.5 / 27.8; 16384, 768 -> 768 40.5 / 50.9; 15313, 1322 ->
+// 64 64.4 / 78.3; 16384, 1600 -> 4800 223 / 236.
+constexpr double kGroupOverhead = 1.0, kGroupSlicesOverhead = 4.0;
+constexpr double kStoreBytesPerUs = 2.5e6, kUnalignedStoreBytesPerUs = 1.0e6;
 
 struct GroupPlan {
     bool grouped;
@@ -1421,7 +1427,8 @@ static GroupPlan grouped_plan(const GemmArgs& dw, const GemmArgs& dx, size_t ws_
     dxs.ws_bytes = dws.ws_bytes = ws_bytes;
     const NtPlan px = nt_plan(dxs);
     if (px.split > 1) return GroupPlan{false, 1, nk0};
-    const double separate = px.cost + nt_plan(dws).cost;
+    const double stores = 2.0 * dx.M * dx.N / (dx.N % 8 == 0 ? kStoreBytesPerUs : kUnalignedStoreBytesPerUs) / kStepUs;
+    const double separate = std::max(px.cost, stores) + nt_plan(dws).cost;
     const int64_t t0 = (int64_t)((dw.M + kPBM - 1) / kPBM) * ((dw.N + kPBN - 1) / kPBN);
     const int64_t t1 = (int64_t)((dx.M + kPBM - 1) / kPBM) * ((dx.N + kPBN - 1) / kPBN);
     GroupPlan best{true, 1, nk0};

@@ -333,6 +333,7 @@ def test_grouped_backward_shapes(dev, M, K, N):
 # the times stand beside the rule in csrc/gemm_fp8.hip)
 @pytest.mark.parametrize("M,K,N,grouped", [(16009, 128, 192, False), (16384, 256, 256, False), (4096, 640, 640, False),
                                            (344, 1941, 136, False), (16384, 768, 768, True), (5000, 1037, 771, True),
+                                           (15313, 1322, 64, True), (8070, 3456, 81, True),
                                            (16384, 1600, 4800, True)])
 def test_backward_takes_the_faster_form(dev, M, K, N, grouped):
     """The grouped launch is priced against the two launches that the
