@@ -10,6 +10,8 @@
 // a type at dnn/core/tensor.cu:489-498).  Semantics: include/df_capi.h.
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -1479,6 +1481,18 @@ __global__ __launch_bounds__(kThreads) void quantize_2d_small_kernel(const InT* 
 // 35.5 against 32.5 us.
 constexpr int kSmallTiles = 256;
 
+// Tile rows up to which the first row of tile blocks adds up the column sums,
+// by the strips (of kT2 columns) of the matrix.  It is a chain of about 31 ns a
+// tile row in one block per strip, which the pass, 12 ns a tile (twice that in
+// fp32), hides from the third strip on.  Longer, narrower matrices take the
+// reduce launch (10 ns a tile row).  us a call, chain / launch: 65536 x 128 bf16
+// (512 tile rows) 22.2 / 18.1, 45000 x 128 (352) 18.9 / 18.8, 1000000 x 64 226 /
+// 145; two strips, 110000 x 200 f16 (860) with both codes 66.0 / 67.5, 1000000 x
+// 200 bf16 468 / 414; fp32, 150000 x 256 84.2 / 88.1.
+static int chain_tiles(int strips, int esz) {
+    return strips == 1 ? 384 : strips == 2 && esz == 2 ? 1024 : INT_MAX;
+}
+
 template <typename InT, int FMT>
 static void launch_q2d_small(hipStream_t st, const InT* x, int rows, int cols, uint8_t* q, int ldq, uint8_t* qt,
                              int ldqt, const JitScale& jit) {
@@ -2025,7 +2039,11 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
         const bool scan = !colsum && n * esz <= kJitScanBytes && (int64_t)grid.x * grid.y <= kSmallTiles;
         if (n > 0 && !scan) {
             if (colsum) {
-                J.nparts = (int)std::min<int64_t>(kJitParts, (int64_t)tile_rows * ((cols + kT2 - 1) / kT2));
+                // one strip: its tiles are few, and partly empty, so every one may have
+                // a block (1000000 x 33 fp32, with the reduce launch: 272 -> 207 us)
+                const int strips = (cols + kT2 - 1) / kT2;
+                J.nparts = (int)std::min<int64_t>(strips == 1 ? kMaxReduceBlocks : kJitParts,
+                                                  (int64_t)tile_rows * strips);
 #define DF_ACS(T)                                                                                             \
     absmax_colsum_stage1<T><<<J.nparts, kThreads, 0, st>>>(static_cast<const T*>(x), rows, cols, vec_ok,      \
                                                            jparts, part)
@@ -2033,7 +2051,7 @@ static int quantize_2d_impl(const char* name, int in_dtype, const void* x, int r
                 else if (in_dtype == DF_DTYPE_HALF) DF_ACS(f16_t);
                 else DF_ACS(uint16_t);
 #undef DF_ACS
-                if (reduce) {  // by the first row of tile blocks
+                if (reduce && tile_rows <= chain_tiles(strips, esz)) {  // by the first row of tile blocks
                     J.colpart = part;
                     J.colsum = colsum;
                     J.tile_rows = tile_rows;

@@ -71,6 +71,26 @@ def test_edges(dev, rows, cols, dt, fmt):
     check(*df.quantize_2d(wide[:, :cols], sc, fmt, want_qt=True))
 
 
+# tile rows (of 128) on and past the counts from which the column sums of a
+# matrix of one or two strips of 128 columns are added up by a launch of their own
+@pytest.mark.parametrize("rows,cols,dt", [(49152, 3, BF16), (49153, 3, F16), (49153, 128, F32), (262145, 9, BF16),
+                                          (131072, 130, BF16), (131073, 130, BF16), (131073, 129, F32)])
+def test_tall_column_sums(dev, rows, cols, dt):
+    """Either way the sums are those of df_quantize_2d_colsum, bit for bit,
+    and absmax, scale and codes those of the calls without sums."""
+    x = tensor(rows, cols, dt, dev, rows + cols)
+    x = torch.where(torch.isfinite(x), x, torch.zeros_like(x))
+    am, sc, q, qt, cs = df.quantize_2d_jit(x, Fmt.E5M2, want_qt=True, colsum=True)
+    am1, sc1 = df.absmax_scale(x, Fmt.E5M2)
+    q1, qt1, cs1 = df.quantize_2d(x, sc1, Fmt.E5M2, want_qt=True, colsum=True)
+    assert am.item() == am1.item() == x.float().abs().max().item() and sc.item() == sc1.item()
+    assert torch.equal(q, q1) and torch.equal(qt, qt1)
+    assert torch.equal(cs.view(torch.int32), cs1.view(torch.int32))
+    ref = x.double().sum(0)
+    bound = rows * 2.0 ** -24 * x.double().abs().sum(0)
+    assert bool(((cs.double() - ref).abs() <= bound).all())
+
+
 # rows of whole 16-byte chunks below, at and past what a wave's registers hold,
 # row counts that leave waves with fewer rows than their share, rows too wide
 # for the registers in whole and part rounds of sixteen values a lane
